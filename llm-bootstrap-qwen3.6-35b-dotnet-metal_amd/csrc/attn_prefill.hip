@@ -1183,11 +1183,16 @@ const char *launch_prefill(Context &c, const View *b, const boot_kernel_args &a,
     // FP16-KV control runs the same schedule with FP16 staging, so that the two differ only in
     // the cache they read.
     p.tiles = (uint32_t)((rows * 8 + kTileRows - 1) / kTileRows);
-    // split-K: enough blocks to fill the CUs, each split at least 256 keys
+    // split-K: as many splits as one round of work-groups on the CUs holds (one per CU; a few blocks
+    // in a second round double the time: 15 row tiles over 8500 keys in 9 splits of 270 blocks), each
+    // at least one key tile. A launch costs about 17 us beyond its 2 us per key tile, so short ranges
+    // gain down to a tile or two per split: attention + combine, same box, (256 rows, no history)
+    // 1 split 37.9, 2 25.5, 8 22.9 us; (512 rows after 512 keys) 4 splits 39.8, 8 33.7; (476 after
+    // 1024) 5 splits 44.6, 8 38.1, 10 (two rounds) 55.8; (300 after 2100) 9 splits 43.7, 12 40.3, 16
+    // (two rounds) 56.2 us. The partials stay below one per CU (64.8 MiB on 256 CUs).
     const uint64_t base_blocks = 2ull * p.tiles;
-    const uint64_t want = (uint64_t)std::max(1, context_cus(c));
-    uint64_t splits = std::max<uint64_t>(1, (want + base_blocks - 1) / base_blocks);
-    splits = std::min<uint64_t>(splits, std::max<uint64_t>(1, keys / 256));
+    const uint64_t round = (uint64_t)std::max(1, context_cus(c));
+    uint64_t splits = std::max<uint64_t>(1, std::min<uint64_t>(round / base_blocks, keys / kW64Keys));
     uint64_t split_keys = (keys + splits - 1) / splits;
     split_keys = (split_keys + kW64Keys - 1) / kW64Keys * kW64Keys;
     splits = (keys + split_keys - 1) / split_keys;
