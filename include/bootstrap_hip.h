@@ -104,7 +104,7 @@ int boot_read(void *ctx, void *buf, uint64_t offset, void *host, uint64_t bytes)
  * (tight serving loops, harnesses that forbid hipMalloc). ----
  *
  * boot_dispatch with the same arguments and outputs, except that kernels whose launch needs
- * scratch (split-K partials of attention_decode_int8, attention_decode_append_int8, the
+ * scratch (split-K partials of attention_decode_int8, attention_verify_int8, attention_decode_append_int8, the
  * attention_online_* prefill names and batch_attention_values_int8; the chunk statistics of
  * attention_softmax) draw it from a static 72 MiB device array of the library instead of the
  * context workspace; it calls no hipMalloc/hipFree or other allocating routine and records no

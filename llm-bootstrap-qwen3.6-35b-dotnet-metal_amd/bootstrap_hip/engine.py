@@ -32,6 +32,7 @@ ATTENTION_WORKSPACE_FLOATS = 32 * 1024 * 1024
 FULL_ATTENTION_LAYERS = tuple(l for l in range(40) if (l + 1) % 4 == 0)
 KV_HEADS, HEAD_DIM, Q_HEADS, GROUP = 2, 256, 16, 8
 ROPE_THETA = 10_000_000.0
+VERIFY_ROWS = 64   # rows of one attention_verify_int8 dispatch at most
 
 
 class ContextLimits:
@@ -445,14 +446,21 @@ def verify_slices(rows: int, position: int,
 def verify_attention_int8(device: Device, layer: Int8KvLayer, rotated: GpuBuffer, gate: GpuBuffer,
                           scores: GpuBuffer, rows: int, position: int,
                           workspace_floats: int = ATTENTION_WORKSPACE_FLOATS) -> None:
-    """INT8 attention of a speculative verify block (Prefill.cs:269-285, ``verify`` true): the
-    scalar reader over query slices. Each slice keeps its absolute causal position and the whole
-    block's key count as the score stride, and writes its output over its own rotated query rows.
-    Inside a command."""
+    """INT8 attention of a speculative verify block (Prefill.cs:269-285, ``verify`` true). Each row
+    keeps its absolute causal position and its output is written over its own rotated query row.
+    ``scores`` is scratch, at least one query slice of ``workspace_floats``. Up to 64 rows inside the
+    window take one dispatch, whose rows do not depend on each other (so neither on the slicing);
+    anything else the scalar reader, slice by slice. Inside a command."""
     length = position + rows
-    for first, count in verify_slices(rows, position, workspace_floats):
-        if scores.length < count * 16 * length * 4:
-            raise ValueError("score workspace smaller than one slice")
+    slices = verify_slices(rows, position, workspace_floats)
+    if scores.length < slices[0][1] * 16 * length * 4:
+        raise ValueError("score workspace smaller than one slice")
+    if rows <= VERIFY_ROWS and length <= NATIVE_WINDOW:
+        p = KernelArgs(M=rows, K=length, Position=position)
+        device.dispatch("attention_verify_int8", p, rows * 4096, 256, rotated, layer.key, layer.value, gate, rotated,
+                        layer.key_scale, layer.value_scale)
+        return
+    for first, count in slices:
         p = KernelArgs(M=count, K=length, Position=position + first)
         query, g = rotated.at(first * 4096 * 4), gate.at(first * 4096 * 4)
         device.dispatch2d("batch_attention_scores_int8", p, length * 32, count * 16, 128, query, layer.key, scores,

@@ -1,6 +1,6 @@
 // Single-token (and 1-8 row verification) INT8 attention over the KV cache.
 //
-// Two entry points:
+// Three entry points:
 //   * the reference's three-kernel reader (kernels.metal:147-156,163-166):
 //     batch_attention_scores_int8 -> attention_softmax -> batch_attention_values_int8,
 //     FP32 scores in a caller buffer; serves serial decode and speculative
@@ -17,6 +17,8 @@
 //     they lie in [0, 1]) split into FP16 hi + lo. Scales are applied to scores
 //     and probabilities as the reference does (score = dot * ks[t] / 16,
 //     P = p * vs[t]).
+//   * attention_verify_int8: the same arithmetic for the rows of a verify block, several
+//     rows per work-group (rows_int8_kernel).
 #include "common.h"
 #include <type_traits>
 #include "kvmath.h"
@@ -1126,6 +1128,440 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float *__rest
     }
 }
 
+// ---------------------------------------------------------------- several rows per work-group
+
+// Attention of up to 2 CT rows against one staging of the keys: verify blocks (FP32 query). The
+// decode kernel above gives each row a work-group of its own, so R rows read, stage and convert
+// the cache R times, and the three-kernel reader (five launches) writes every score to memory and
+// reads it back twice. Per layer, with the combine, against the reader: 8 rows after 1500 keys 14.9
+// (40.0) us, where either is launches and one chunk's latency; 4 rows after 30000 keys 24.4 (47.6)
+// us, 1.3 TB/s of cache: bound by the vector work of a chunk (conversions, exponentials, P) and the
+// start of a work-group, not by the stream.
+//
+// Grid: (split, KV group) pairs x row blocks, one 8-wave work-group per CU; the row blocks of a pair
+// are 8 blocks apart, on one XCD, whose L2 serves the second and later ones. A split is split_chunks
+// chunks of 128 tokens, streamed as in decode_int8_kernel, with the same arithmetic (three INT8
+// query parts, FP16 hi + lo probabilities, lazy running maxima), and these differences:
+//   * 16 MFMA columns are two rows x 8 heads, for each of q1, q2, q3 (the three parts of a score meet
+//     in one lane) and for P's hi and lo parts (which accumulate into one O), so no column computes
+//     another's exponentials and nothing is exchanged between column halves;
+//   * wave w stages its own 16 K rows in an LDS slice that no other wave reads (whole 256-byte rows
+//     per load, no barrier); V and P are shared as there;
+//   * every quantity of a column (its running maximum and rescales, its V scale reference over the
+//     tokens it sees) depends on that row alone, and split boundaries are absolute, so a row's result
+//     does not depend on the rows dispatched with it: a verify block's rows are bitwise those of any
+//     shorter block or slice.
+// 4 rows keep two of their three query parts in 64 registers, the third in LDS; 8 rows would need
+// twice that, and 64 KB of LDS for their P operands beside the 112 KB of staging and scales.
+struct RowsParams {
+    const float *q;   // FP32 [rows][16][256]
+    const int8_t *k;
+    const int8_t *v;
+    const float *ks;
+    const float *vs;
+    const float *gate;
+    float *y;
+    float *partial;   // as decode_int8_kernel's
+    uint32_t rows, pos, splits, split_chunks, zs;   // zs: row blocks
+};
+
+template <int CT, bool kOnce>
+__global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    constexpr int kRowsPer = 2 * CT;
+    __shared__ uint4 vbuf[2][256][8];                        // V chunks by parity, as ChunkLds::v
+    __shared__ uint4 kbuf[kDecodeWaves][16][16];             // each wave's K rows, piece c of row t at c ^ t
+    __shared__ uint2 pshare[2][CT][2][kDecodeWaves][64];     // P operands [parity][tile][hi, lo][wave][lane]
+    __shared__ __attribute__((aligned(16))) float kscale[kMaxSplitTokens], vscale[kMaxSplitTokens];
+    __shared__ float chunk_top[2][CT][kDecodeWaves][16], wave_l[CT][kDecodeWaves][16];
+    __shared__ float red[kDecodeWaves], qmax[CT][4][16];
+    // the query operands [tile][part][64-dimension step][lane]: q1 and q2, built once and read into
+    // registers, in V buffer 1, which is first written in phase 1, after the barrier that ends phase 0;
+    // q3 stays in LDS (in registers it spilled, and a reload waits for the chunk loads before it)
+    v4i(*qlds)[2][4][64] = reinterpret_cast<v4i(*)[2][4][64]>(&vbuf[1][0][0]);
+    static_assert(CT * 2 * 4 * 64 * sizeof(v4i) <= sizeof(vbuf[0]), "query operands exceed a V buffer");
+    __shared__ v4i q3lds[CT][4][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = lane & 15, qq = lane >> 4, head = n & 7;
+    const uint32_t xcd = blockIdx.x % 8, jb = blockIdx.x / 8, pair = (jb / p.zs) * 8 + xcd;
+    if (pair >= 2 * p.splits) return;   // padding of the grid to whole rounds of 8
+    const uint32_t split = pair >> 1, g = pair & 1, r0 = (jb % p.zs) * kRowsPer;
+    const uint32_t nr = min((uint32_t)kRowsPer, p.rows - r0);
+    const uint32_t first_end = p.pos + r0 + 1, block_end = p.pos + r0 + nr;   // keys of the first and last row
+    const uint32_t begin = split * p.split_chunks * kChunk;
+    const uint32_t end = min(block_end, begin + p.split_chunks * kChunk);
+    auto part_of = [&](uint32_t ri) __attribute__((always_inline)) {
+        return p.partial + (((size_t)(r0 + ri) * 2 + g) * p.splits + split) * kPartialFloats;
+    };
+    if (begin >= block_end) {   // no keys of these rows (only with several splits): an empty partial
+        if (tid < 8 * (int)nr) part_of(tid >> 3)[2048 + (tid & 7)] = -INFINITY;
+        return;
+    }
+    const uint32_t nchunks = (end - begin + kChunk - 1) / kChunk;
+
+    // ---- the small loads first, then the first two chunks (as decode_int8_kernel)
+    const uint32_t last = end - 1;
+    float ksv[kMaxSplitTokens / 512], vsv[kMaxSplitTokens / 512], vnew[kRowsPer];
+#pragma unroll
+    for (int it = 0; it < kMaxSplitTokens / 512; it++) {
+        const size_t at = (size_t)min(begin + tid + 512 * it, last) * 2 + g;
+        ksv[it] = p.ks[at];
+        vsv[it] = p.vs[at];
+    }
+    // the V scales of the tokens between the first and the last row's ends
+#pragma unroll
+    for (int i = 0; i + 1 < kRowsPer; i++) vnew[i] = p.vs[(size_t)min(first_end + i, last) * 2 + g];
+    const int qct = CT == 2 ? wave >> 2 : 0, chunk = wave & 3;   // the query tile and step this wave builds
+    float4 x[4];
+    {
+        const uint32_t row = r0 + min((uint32_t)(2 * qct + (n >> 3)), nr - 1);
+        const float *qs = p.q + ((size_t)row * 16 + g * 8 + head) * 256 + 64 * chunk + 16 * qq;
+#pragma unroll
+        for (int f = 0; f < 4; f++) x[f] = *reinterpret_cast<const float4 *>(qs + 4 * f);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    // kOnce: the codes are read by this work-group only (one row block) and need not stay in L2
+    auto load16 = [&](const int8_t *at) __attribute__((always_inline)) {
+        if constexpr (kOnce) return load_piece(at);
+        return *reinterpret_cast<const uint4 *>(at);
+    };
+    // K rows 16 wave + 4 i + lane / 16 of chunk idx, piece lane % 16; V segments as load_v. Past the
+    // last chunk (only the prologue's second load) every lane reads one line of the first.
+    auto load_k = [&](KRegs &r, uint32_t idx) __attribute__((always_inline)) {
+        const bool real = idx < nchunks;
+        const uint32_t t = begin + (real ? idx * kChunk + 16 * wave + (lane >> 4) : 0u), step = real ? 4 : 0;
+        const int8_t *base = p.k + (size_t)g * 256 + 16 * (real ? lane & 15 : 0);
+        r.k0 = load16(base + (size_t)min(t, last) * 512);
+        r.k1 = load16(base + (size_t)min(t + step, last) * 512);
+        r.k2 = load16(base + (size_t)min(t + 2 * step, last) * 512);
+        r.k3 = load16(base + (size_t)min(t + 3 * step, last) * 512);
+    };
+    auto load_v = [&](VRegs &r, uint32_t idx) __attribute__((always_inline)) {
+        const bool real = idx < nchunks;
+        const uint32_t c0 = begin + (real ? idx * kChunk : 0u);
+        const int lt = real ? tid : 0;
+        const int8_t *vrow = p.v + value_index((uint64_t)c0 * 2 + g, 0) + (size_t)(lt >> 3) * 256 + 16 * (lt & 7);
+        const size_t step = real ? 64 * 256 : 0;
+        r.v0 = load16(vrow);
+        r.v1 = load16(vrow + step);
+        r.v2 = load16(vrow + 2 * step);
+        r.v3 = load16(vrow + 3 * step);
+    };
+    auto store_k = [&](const KRegs &r) __attribute__((always_inline)) {
+        const int t = lane >> 4, c = lane & 15;
+        kbuf[wave][t][c ^ t] = r.k0;
+        kbuf[wave][t + 4][c ^ (t + 4)] = r.k1;
+        kbuf[wave][t + 8][c ^ (t + 8)] = r.k2;
+        kbuf[wave][t + 12][c ^ (t + 12)] = r.k3;
+    };
+    auto store_v = [&](int slot, const VRegs &r) __attribute__((always_inline)) {
+        const int d = tid >> 3, vp = (tid & 7) ^ ((d >> 1) & 7);   // V rows d + 64 i (same (d / 2) % 8)
+        vbuf[slot][d][vp] = r.v0;
+        vbuf[slot][d + 64][vp] = r.v1;
+        vbuf[slot][d + 128][vp] = r.v2;
+        vbuf[slot][d + 192][vp] = r.v3;
+    };
+    KRegs ka, kb;   // K of even / odd chunks
+    VRegs va, vb;   // V of even / odd chunks
+    load_k(ka, 0);
+    load_v(va, 0);
+    load_k(kb, 1);
+    load_v(vb, 1);
+
+    // ---- scales of the split into LDS, the columns' V scale references, the query's INT8 parts
+    float vmax = 0.0f;
+#pragma unroll
+    for (int it = 0; it < kMaxSplitTokens / 512; it++) {
+        const uint32_t e = tid + 512 * it, t = begin + e;
+        kscale[e] = t < end ? ksv[it] * (kLog2e / 16.0f) : 0.0f;
+        vscale[e] = t < end ? vsv[it] : 0.0f;
+        vmax = fmaxf(vmax, t < min(end, first_end) ? vsv[it] : 0.0f);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
+    if (lane == 0) red[wave] = vmax;
+    float amax = 0.0f;
+#pragma unroll
+    for (int f = 0; f < 4; f++) amax = fmaxf(amax, fmaxf(fmaxf(fabsf(x[f].x), fabsf(x[f].y)), fmaxf(fabsf(x[f].z), fabsf(x[f].w))));
+    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+    if (lane < 16 && wave < 4 * CT) qmax[qct][chunk][lane] = amax;
+    __syncthreads();
+    // row i of the block sees the tokens before first_end and vnew[0 .. i - 1], where the split holds them
+    float vcum = red[0];
+#pragma unroll
+    for (int w = 1; w < kDecodeWaves; w++) vcum = fmaxf(vcum, red[w]);
+    float vref[CT], vinv[CT], qsc[CT];
+    uint32_t row_end[CT];   // keys the column's row sees (a missing row repeats the last one)
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        float two[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int ri = 2 * ct + i;
+            if (ri > 0) {
+                const uint32_t t = first_end + ri - 1;
+                vcum = fmaxf(vcum, t >= begin && t < end ? vnew[ri - 1] : 0.0f);
+            }
+            two[i] = vcum;
+        }
+        const float even = two[0], odd = two[1];
+        vref[ct] = n >= 8 ? odd : even;
+        // operands up to 2^8 times 2^7 stay below FP16's 65504; the factor keeps their lo parts out of
+        // its subnormals
+        vinv[ct] = vref[ct] > 0.0f ? 128.0f / vref[ct] : 0.0f;
+        vref[ct] *= 1.0f / 128.0f;
+        qsc[ct] = fmaxf(fmaxf(qmax[ct][0][n], qmax[ct][1][n]), fmaxf(qmax[ct][2][n], qmax[ct][3][n])) * (1.0f / 127.0f);
+        row_end[ct] = first_end + min((uint32_t)(2 * ct + (n >> 3)), nr - 1);
+    }
+    {
+        const float qabs = fmaxf(fmaxf(qmax[qct][0][n], qmax[qct][1][n]), fmaxf(qmax[qct][2][n], qmax[qct][3][n]));
+        const float inv = qabs > 0.0f ? 127.0f / qabs : 0.0f;
+        auto code = [](float q) { return (uint32_t)(uint8_t)(int8_t)(int)fminf(fmaxf(q, -127.0f), 127.0f); };
+        uint32_t w1[4], w2[4], w3[4];
+#pragma unroll
+        for (int f = 0; f < 4; f++) {
+            const float xs[4] = {x[f].x, x[f].y, x[f].z, x[f].w};
+            w1[f] = w2[f] = w3[f] = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {   // as decode_int8_kernel
+                const float z = xs[e] * inv, q1 = rintf(z), r1 = z - q1;
+                const float q2 = rintf(r1 * 254.0f);
+                const float r2 = fmaf(r1, 254.0f, -q2);
+                const float q3 = rintf(r2 * 254.0f);
+                w1[f] |= code(q1) << (8 * e);
+                w2[f] |= code(q2) << (8 * e);
+                w3[f] |= code(q3) << (8 * e);
+            }
+        }
+        if (wave < 4 * CT) {
+            qlds[qct][0][chunk][lane] = v4i{(int)w1[0], (int)w1[1], (int)w1[2], (int)w1[3]};
+            qlds[qct][1][chunk][lane] = v4i{(int)w2[0], (int)w2[1], (int)w2[2], (int)w2[3]};
+            q3lds[qct][chunk][lane] = v4i{(int)w3[0], (int)w3[1], (int)w3[2], (int)w3[3]};
+        }
+    }
+    store_k(ka);
+    if (2 < nchunks) load_k(ka, 2);
+    __syncthreads();
+    v4i qi[CT][2][4];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int part = 0; part < 2; part++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) qi[ct][part][c] = qlds[ct][part][c][lane];
+
+    floatx4 o[2][CT];   // O^T: dimensions 32 wave + 16 dt + 4 qq + r of column n
+    float m[CT], l[CT], total_prev[CT], dot_prev[CT][4];   // l: this lane's tokens, summed over lanes at the end
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        o[0][ct] = o[1][ct] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        m[ct] = -INFINITY;
+        l[ct] = total_prev[ct] = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; r++) dot_prev[ct][r] = 0.0f;
+    }
+    int local_prev = 0;
+    auto probs = [&](int slot) __attribute__((always_inline)) {
+        const float4 vs4 = *reinterpret_cast<const float4 *>(&vscale[local_prev]);
+        const float4 ks4 = *reinterpret_cast<const float4 *>(&kscale[local_prev]);
+        const float vsr[4] = {vs4.x, vs4.y, vs4.z, vs4.w}, ksr[4] = {ks4.x, ks4.y, ks4.z, ks4.w};
+        const uint32_t t0 = begin + (uint32_t)local_prev;
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+            // m = -inf (before the column's first rescale): its operands are rebuilt before they are read
+            const float refc = fmaxf(m[ct], -3.0e38f);
+            half4 hi, lo;
+            float total = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float arg = fmaf(dot_prev[ct][r], qsc[ct] * ksr[r], -refc);
+                const float prob = __builtin_amdgcn_exp2f(t0 + r < row_end[ct] ? arg : -INFINITY);
+                total += prob;
+                float scaled = prob * (vsr[r] * vinv[ct]);
+                // one rounded FP32 value: else the operand's hi is the exact product rounded once
+                // (v_fma_mixlo_f16) and the hi that lo completes the rounded product rounded again,
+                // which differ by 2^-10 in rare near-ties
+                asm("" : "+v"(scaled));
+                hi[r] = (_Float16)scaled;
+                lo[r] = (_Float16)(scaled - (float)hi[r]);
+            }
+            total_prev[ct] = total;
+            pshare[slot][ct][0][wave][lane] = __builtin_bit_cast(uint2, hi);
+            pshare[slot][ct][1][wave][lane] = __builtin_bit_cast(uint2, lo);
+        }
+    };
+    // the phases of decode_int8_kernel: finish chunk j - 1, score chunk j, stage V of chunk j and K of
+    // chunk j + 1, load V of chunk j + 2 and K of chunk j + 3; one barrier each
+    auto finish = [&](uint32_t j) __attribute__((always_inline)) {
+        const int slot = (j - 1) & 1;
+        float ctop[CT];
+        bool raise = false;
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+            ctop[ct] = chunk_top[slot][ct][0][n];
+#pragma unroll
+            for (int w = 1; w < kDecodeWaves; w++) ctop[ct] = fmaxf(ctop[ct], chunk_top[slot][ct][w][n]);
+            raise |= ctop[ct] > m[ct] + 8.0f;
+        }
+        // every wave reads the same maxima: the branch is uniform over the work-group. Only the
+        // columns that passed the bound change (the others' factor is 1 and their operands the same)
+        if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++) {
+                const float next = ctop[ct] > m[ct] + 8.0f ? ctop[ct] : m[ct];
+                const float decay = next == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[ct] - next);
+                l[ct] *= decay;
+                o[0][ct] *= decay;
+                o[1][ct] *= decay;
+                m[ct] = next;
+            }
+            probs(slot);
+            __syncthreads();
+        }
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) l[ct] += total_prev[ct];
+#pragma unroll
+        for (int s = 0; s < kDecodeWaves / 2; s++) {
+            const int src = 2 * s + (qq >> 1), at = n + 32 * (qq & 1);
+            half8 ps[CT][2];
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+                for (int hl = 0; hl < 2; hl++) {
+                    const uint2 pa = pshare[slot][ct][hl][src][at], pb = pshare[slot][ct][hl][src][at + 16];
+                    ps[ct][hl] = __builtin_bit_cast(half8, make_uint4(pa.x, pa.y, pb.x, pb.y));
+                }
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++) {
+                const int d = 16 * (2 * wave + dt) + n;
+                const uint2 w8 = reinterpret_cast<const uint2 *>(&vbuf[slot][d][src ^ ((d >> 1) & 7)])[qq & 1];
+                uint32_t h0, h1, h2, h3;
+                i8x8_to_f16_sdwa(w8.x, w8.y, h0, h1, h2, h3);
+                const half8 va8 = __builtin_bit_cast(half8, make_uint4(h0, h1, h2, h3));
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) {
+                    o[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va8, ps[ct][0], o[dt][ct], 0, 0, 0);
+                    o[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va8, ps[ct][1], o[dt][ct], 0, 0, 0);
+                }
+            }
+        }
+    };
+    auto phase = [&](uint32_t j, auto odd, bool store_knext, bool load_v2, bool load_k3) __attribute__((always_inline)) {
+        VRegs &rv = decltype(odd)::value ? vb : va;
+        KRegs &rk = decltype(odd)::value ? ka : kb;
+        if (j > 0) finish(j);
+        {
+            v4i acc[CT][3];
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+                for (int part = 0; part < 3; part++) acc[ct][part] = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) {
+                const v4i kop = __builtin_bit_cast(v4i, kbuf[wave][n][(4 * jj + qq) ^ n]);
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) {
+                    acc[ct][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, qi[ct][0][jj], acc[ct][0], 0, 0, 0);
+                    acc[ct][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, qi[ct][1][jj], acc[ct][1], 0, 0, 0);
+                    acc[ct][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, q3lds[ct][jj][lane], acc[ct][2], 0, 0, 0);
+                }
+            }
+            const int local0 = (int)(j * kChunk) + 16 * wave + 4 * qq;   // token offset inside the split
+            const uint32_t t0 = begin + (uint32_t)local0;
+            const float4 ks4 = *reinterpret_cast<const float4 *>(&kscale[local0]);
+            const float ksr[4] = {ks4.x, ks4.y, ks4.z, ks4.w};
+            local_prev = local0;
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++) {
+                float top = -INFINITY;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    // every dot is an integer below 2^22 in magnitude, exact in FP32. The exponent's
+                    // argument is one fma of the dot (probs), so the score itself, rounded, is only
+                    // compared
+                    const float full = fmaf((float)acc[ct][2][r], 1.0f / 64516.0f,
+                                            fmaf((float)acc[ct][1][r], 1.0f / 254.0f, (float)acc[ct][0][r]));
+                    dot_prev[ct][r] = full;
+                    top = fmaxf(top, t0 + r < row_end[ct] ? full * (qsc[ct] * ksr[r]) : -INFINITY);
+                }
+                top = xl_max16(top);
+                top = xl_max32(top);
+                if (qq == 0) chunk_top[j & 1][ct][wave][n] = top;
+            }
+            probs(j & 1);
+        }
+        store_v(j & 1, rv);
+        if (load_v2) load_v(rv, j + 2);
+        if (store_knext) store_k(rk);
+        if (load_k3) load_k(rk, j + 3);
+        __syncthreads();
+    };
+    uint32_t c = 0;
+    for (; c + 4 < nchunks; c += 2) {
+        phase(c, std::false_type{}, true, true, true);
+        phase(c + 1, std::true_type{}, true, true, true);
+    }
+    phase(c, std::false_type{}, c + 1 < nchunks, c + 2 < nchunks, c + 3 < nchunks);
+    uint32_t last_phase = c + 1;
+    if (c + 1 < nchunks) {
+        phase(c + 1, std::true_type{}, c + 2 < nchunks, c + 3 < nchunks, false);
+        last_phase = c + 2;
+        if (c + 2 < nchunks) {
+            phase(c + 2, std::false_type{}, c + 3 < nchunks, false, false);
+            last_phase = c + 3;
+            if (c + 3 < nchunks) {
+                phase(c + 3, std::true_type{}, false, false, false);
+                last_phase = c + 4;
+            }
+        }
+    }
+    finish(last_phase);
+
+    // ---- l over the lanes and waves; O^T[d][n] times the column's V scale reference
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        const float lt = xl_sum32(xl_sum16(l[ct]));
+        if (qq == 0) wave_l[ct][wave][n] = lt;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        const uint32_t ri = 2 * ct + (n >> 3);
+        if (ri >= nr) continue;
+        float lw = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kDecodeWaves; w++) lw += wave_l[ct][w][n];
+        if (p.splits == 1) {
+            const float inv = 1.0f / lw;
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++) {
+                // gate and y need only 4-byte alignment (the gate loads go out before the first store)
+                const size_t at = ((size_t)(r0 + ri) * 16 + g * 8 + head) * 256 + 32 * wave + 16 * dt + 4 * qq;
+                const float g0 = p.gate[at + 0], g1 = p.gate[at + 1], g2 = p.gate[at + 2], g3 = p.gate[at + 3];
+                asm volatile("" ::"v"(g0), "v"(g1), "v"(g2), "v"(g3) : "memory");
+                p.y[at + 0] = o[dt][ct][0] * vref[ct] * inv * sigmoidf(g0);
+                p.y[at + 1] = o[dt][ct][1] * vref[ct] * inv * sigmoidf(g1);
+                p.y[at + 2] = o[dt][ct][2] * vref[ct] * inv * sigmoidf(g2);
+                p.y[at + 3] = o[dt][ct][3] * vref[ct] * inv * sigmoidf(g3);
+            }
+            continue;
+        }
+        float *part = part_of(ri);
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++)
+            *reinterpret_cast<float4 *>(part + head * 256 + 32 * wave + 16 * dt + 4 * qq) =
+                make_float4(o[dt][ct][0] * vref[ct], o[dt][ct][1] * vref[ct], o[dt][ct][2] * vref[ct], o[dt][ct][3] * vref[ct]);
+        if (wave == 0 && qq == 0) {
+            part[2048 + head] = m[ct];
+            part[2056 + head] = lw;
+        }
+    }
+}
+
 inline bool aligned(const void *p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 }  // namespace
@@ -1341,6 +1777,73 @@ const char *launch_decode_int8(Context &c, const View *b, int count, const boot_
     d.k_out = d.v_out = nullptr;
     d.ks_out = d.vs_out = nullptr;
     return decode_launch(c, d, rows, length);
+}
+
+const char *launch_verify_int8(Context &c, const View *b, int count, const boot_kernel_args &p, const uint32_t *) {
+    // bindings (attention_decode_int8's order): q FP32 [rows][16][256] (rotated), k, v, gate, y, ks, vs.
+    // Row r attends t <= pos + r; its result depends on that row alone, and y may be q.
+    BOOT_REQUIRE(count >= 7, "attention_verify_int8 needs 7 bindings: q, k, v, gate, y, ks, vs");
+    const uint64_t rows = p.m;
+    if (rows == 0) return nullptr;
+    BOOT_REQUIRE(rows <= 64, "attention_verify_int8 serves at most 64 rows");
+    const uint64_t length = (uint64_t)p.pos + rows;
+    BOOT_REQUIRE(length <= 262144, "attended length exceeds the 262144-token window");
+    BOOT_REQUIRE(b[0].bytes >= rows * 16384, "query buffer smaller than rows*4096 floats");
+    BOOT_REQUIRE(b[1].bytes >= length * 512, "K cache smaller than the attended length");
+    BOOT_REQUIRE(b[2].bytes >= value_bytes(length), "V cache smaller than whole pages of the attended length");
+    BOOT_REQUIRE(b[3].bytes >= rows * 16384 && b[4].bytes >= rows * 16384, "gate/output smaller than rows*4096 floats");
+    BOOT_REQUIRE(b[5].bytes >= length * 8 && b[6].bytes >= length * 8, "KV scale buffers smaller than the attended length");
+    BOOT_REQUIRE(aligned(b[0].ptr, 16) && aligned(b[1].ptr, 16) && aligned(b[2].ptr, 16) && aligned(b[3].ptr, 4) &&
+                     aligned(b[4].ptr, 4) && aligned(b[5].ptr, 4) && aligned(b[6].ptr, 4),
+                 "bindings misaligned (q, k, v need 16 bytes)");
+    // A row's split is as many chunks as spread its own keys over a number of work-groups per KV
+    // group, whatever rows come with it, so that its result depends on its position alone; rows of
+    // one launch have the same split (a block across a boundary takes two launches). 64 work-groups
+    // up to 65536 keys: with two groups and two row blocks one round of 256 CUs, 8 rows after 9000
+    // keys 19.4 (128 work-groups: 27.8) us, after 30000 24.7 (35.0), where 4 rows lose little, 18.6
+    // (17.3) and 24.4 (24.1) us. 128 beyond, one round for up to 4 rows: 100000 keys 38.4 (64: 46.9)
+    // us, against 63.4 (48.5) us for 8 rows.
+    constexpr uint32_t kNearChunks = 65536 / kChunk, kNearSlots = 64, kFarSlots = 128;
+    auto chunks_of = [&](uint64_t row) { return (uint32_t)(((uint64_t)p.pos + row) / kChunk + 1); };
+    auto split_of = [&](uint64_t row) {
+        const uint32_t chunks = chunks_of(row), slots = chunks <= kNearChunks ? kNearSlots : kFarSlots;
+        return (chunks + slots - 1) / slots;
+    };
+    static_assert(kNearChunks <= kNearSlots * (kMaxSplitTokens / kChunk) &&
+                      262144 / kChunk <= kFarSlots * (kMaxSplitTokens / kChunk), "a split's scales exceed the LDS");
+    for (uint64_t first = 0; first < rows;) {
+        uint64_t next = first + 1;
+        while (next < rows && split_of(next) == split_of(first)) next++;
+        RowsParams d;
+        d.q = (const float *)b[0].ptr + first * 4096;
+        d.k = (const int8_t *)b[1].ptr;
+        d.v = (const int8_t *)b[2].ptr;
+        d.gate = (const float *)b[3].ptr + first * 4096;
+        d.y = (float *)b[4].ptr + first * 4096;
+        d.ks = (const float *)b[5].ptr;
+        d.vs = (const float *)b[6].ptr;
+        d.rows = (uint32_t)(next - first);
+        d.pos = (uint32_t)(p.pos + first);
+        d.split_chunks = split_of(first);
+        d.splits = (chunks_of(next - 1) + d.split_chunks - 1) / d.split_chunks;
+        d.partial = nullptr;
+        if (d.splits > 1) {
+            d.partial = (float *)context_workspace(c, (uint64_t)d.rows * 2 * d.splits * kPartialFloats * sizeof(float));
+            BOOT_REQUIRE(d.partial, "cannot allocate verify split workspace");
+        }
+        // one or two rows: half the columns and registers (1 row after 1500 keys 7.8 against 9.7 us)
+        const bool narrow = d.rows <= 2;
+        d.zs = narrow ? 1 : (d.rows + 3) / 4;
+        const dim3 grid((2 * d.splits + 7) / 8 * 8 * d.zs);
+        launch_timed(c, "rows_int8_kernel",
+                     narrow ? rows_int8_kernel<1, true> : d.zs == 1 ? rows_int8_kernel<2, true> : rows_int8_kernel<2, false>,
+                     grid, dim3(512), d);
+        if (d.splits > 1)
+            launch_timed(c, "decode_combine_kernel", decode_combine_kernel, dim3(4, 16, d.rows), dim3(256),
+                         (const float *)d.partial, d.gate, d.y, d.splits);
+        first = next;
+    }
+    return nullptr;
 }
 
 const char *launch_online_int8_as_decode(Context &c, const View *b, const boot_kernel_args &p) {

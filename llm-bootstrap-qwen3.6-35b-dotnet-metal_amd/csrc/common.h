@@ -91,6 +91,7 @@ const char *launch_decode_int8(Context &, const View *, int, const boot_kernel_a
 // kernel (bindings validated by the prefill launcher)
 const char *launch_online_int8_as_decode(Context &, const View *, const boot_kernel_args &);
 const char *launch_decode_append_int8(Context &, const View *, int, const boot_kernel_args &, const uint32_t *);
+const char *launch_verify_int8(Context &, const View *, int, const boot_kernel_args &, const uint32_t *);
 const char *launch_scores_int8(Context &, const View *, int, const boot_kernel_args &, const uint32_t *);
 const char *launch_softmax(Context &, const View *, int, const boot_kernel_args &, const uint32_t *);
 const char *launch_values_int8(Context &, const View *, int, const boot_kernel_args &, const uint32_t *);
