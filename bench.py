@@ -59,8 +59,9 @@ def upload(device, array):
     return b
 
 
-# the INT8 prefill attention kernel (its FP16-KV control: prefill_w64_fp16_kernel)
-PREFILL_INT8_KERNELS = ["prefill_w64_kernel"]
+# the INT8 prefill attention kernels: the main one (its FP16-KV control: prefill_w64_fp16_kernel) and
+# the multi-row kernel that serves the chunks over the first keys
+PREFILL_INT8_KERNELS = ["prefill_w64_kernel", "rows_int8_half_query_kernel"]
 
 
 def kernel_stats(device, names):
@@ -173,11 +174,11 @@ def reference_shapes(work: PrefillWorkload, runs: int = 20):
             ws.encode_int8(None, layer.key, layer.value, layer.key_scale, layer.value_scale, gate, out, rows, history,
                            prepared_query=True)
         d.end()
-        # chunks of at most 64 rows over a short history run on the decode kernel (its grouped FP16
-        # query variant) and, when split, its combine
-        ks = kernel_stats(d, ["prefill_w64_kernel", "prefill_combine_kernel", "decode_int8_half_query_kernel",
-                              "decode_combine_kernel"])
-        kernel = "prefill_w64_kernel" if "prefill_w64_kernel" in ks else "decode_int8_half_query_kernel"
+        # small chunks run on the decode kernel or the multi-row kernel (their grouped FP16 query
+        # variants) and, when split, their combine
+        served = PREFILL_INT8_KERNELS + ["decode_int8_half_query_kernel"]
+        ks = kernel_stats(d, served + ["prefill_combine_kernel", "decode_combine_kernel"])
+        kernel = next(n for n in served if n in ks)
         attn = ks[kernel][0] / runs
         comb = sum(ks.get(n, (0.0, 0))[0] for n in ("prefill_combine_kernel", "decode_combine_kernel")) / runs
         flops = prefill_flops(history, rows)
@@ -521,11 +522,11 @@ def main():
     attn_kernel = next((k for k in PREFILL_INT8_KERNELS if k in timed), None)
     if attn_kernel is None:
         raise SystemExit("no INT8 prefill attention kernel was timed")
-    ks = kernel_stats(device, [attn_kernel, "prefill_combine_kernel", "prepare_fused_int8_kernel"])
+    ks = kernel_stats(device, ["prefill_combine_kernel", "prepare_fused_int8_kernel"])
     y_int8 = work.out.read(np.float32, work.chunk * 4096)     # the last chunk's INT8 output
-    attn_ms = ks[attn_kernel][0] / args.steps
+    attn_ms = sum(ms for ms, _ in timed.values()) / args.steps
     combine_ms = ks.get("prefill_combine_kernel", (0.0, 0))[0] / args.steps
-    launches = ks[attn_kernel][1] // args.steps
+    launches = sum(n for _, n in timed.values()) // args.steps
     flops = work.flops()
     achieved = flops / (attn_ms * 1e-3) / 1e12
     result = {

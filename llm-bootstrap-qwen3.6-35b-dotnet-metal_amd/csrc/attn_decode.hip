@@ -476,6 +476,23 @@ __device__ inline float xl_swap8(float x) {
     return y;
 }
 
+// Every element's maximum over the wave: rotations of the 16-lane rows by DPP (the steps of
+// several elements interleave, covering each other's wait states), then across the rows
+template <int N>
+__device__ inline void wave_allmax(float (&x)[N]) {
+#pragma unroll
+    for (int step = 0; step < 4; step++)
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            if (step == 0) asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf" : "+v"(x[i]));
+            if (step == 1) asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf" : "+v"(x[i]));
+            if (step == 2) asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:2 row_mask:0xf bank_mask:0xf" : "+v"(x[i]));
+            if (step == 3) asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf" : "+v"(x[i]));
+        }
+#pragma unroll
+    for (int i = 0; i < N; i++) x[i] = xl_max32(xl_max16(x[i]));
+}
+
 __device__ inline float sigmoidf(float x) {
     return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * 1.4426950408889634f));
 }
@@ -1130,7 +1147,8 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float *__rest
 
 // ---------------------------------------------------------------- several rows per work-group
 
-// Attention of up to 2 CT rows against one staging of the keys: verify blocks (FP32 query). The
+// Attention of up to 2 CT rows against one staging of the keys: verify blocks (FP32 query) and
+// prefill chunks over short key ranges (grouped FP16 query). The
 // decode kernel above gives each row a work-group of its own, so R rows read, stage and convert
 // the cache R times, and the three-kernel reader (five launches) writes every score to memory and
 // reads it back twice. Per layer, with the combine, against the reader: 8 rows after 1500 keys 14.9
@@ -1154,7 +1172,8 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float *__rest
 // 4 rows keep two of their three query parts in 64 registers, the third in LDS; 8 rows would need
 // twice that, and 64 KB of LDS for their P operands beside the 112 KB of staging and scales.
 struct RowsParams {
-    const float *q;   // FP32 [rows][16][256]
+    const float *q;         // FP32 [rows][16][256], or
+    const _Float16 *qh;     // kHalfQ: the grouped FP16 query [2][rows][8][256]
     const int8_t *k;
     const int8_t *v;
     const float *ks;
@@ -1165,18 +1184,22 @@ struct RowsParams {
     uint32_t rows, pos, splits, split_chunks, zs;   // zs: row blocks
 };
 
-template <int CT, bool kOnce>
+template <int CT, bool kOnce, bool kHalfQ>
 __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     typedef int v4i __attribute__((ext_vector_type(4)));
     typedef _Float16 half4 __attribute__((ext_vector_type(4)));
     constexpr int kRowsPer = 2 * CT;
     __shared__ uint4 vbuf[2][256][8];                        // V chunks by parity, as ChunkLds::v
     __shared__ uint4 kbuf[kDecodeWaves][16][16];             // each wave's K rows, piece c of row t at c ^ t
-    __shared__ uint2 pshare[2][CT][2][kDecodeWaves][64];     // P operands [parity][tile][hi, lo][wave][lane]
+    // P operands [parity][tile][hi, lo][wave][column][four of the wave's tokens]: a PV step's eight
+    // tokens are one 16-byte read, a wave's reads and writes contiguous
+    __shared__ __attribute__((aligned(16))) uint2 pshare[2][CT][2][kDecodeWaves][16][4];
     __shared__ __attribute__((aligned(16))) float kscale[kMaxSplitTokens], vscale[kMaxSplitTokens];
-    __shared__ float chunk_top[2][CT][kDecodeWaves][16], wave_l[CT][kDecodeWaves][16];
-    __shared__ float red[kDecodeWaves], qmax[CT][4][16];
-    // the query operands [tile][part][64-dimension step][lane]: q1 and q2, built once and read into
+    __shared__ __attribute__((aligned(16))) float chunk_top[2][CT][16][kDecodeWaves];
+    __shared__ float wave_l[CT][kDecodeWaves][16];
+    __shared__ float red[kDecodeWaves], qmax[CT][16];
+    // the query operands [tile][part][64-dimension step c][slot], lane (n, qq)'s in slot
+    // 16 qq + (n ^ (4 c + qq)), so that the 4-byte writes below spread over the banks: q1 and q2, built once and read into
     // registers, in V buffer 1, which is first written in phase 1, after the barrier that ends phase 0;
     // q3 stays in LDS (in registers it spilled, and a reload waits for the chunk loads before it)
     v4i(*qlds)[2][4][64] = reinterpret_cast<v4i(*)[2][4][64]>(&vbuf[1][0][0]);
@@ -1184,9 +1207,17 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     __shared__ v4i q3lds[CT][4][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 15, qq = lane >> 4, head = n & 7;
-    const uint32_t xcd = blockIdx.x % 8, jb = blockIdx.x / 8, pair = (jb / p.zs) * 8 + xcd;
-    if (pair >= 2 * p.splits) return;   // padding of the grid to whole rounds of 8
-    const uint32_t split = pair >> 1, g = pair & 1, r0 = (jb % p.zs) * kRowsPer;
+    uint32_t pair, zb;
+    if constexpr (kHalfQ) {   // pairs in turn: few pairs and many row blocks must reach every XCD
+        pair = blockIdx.x % (2 * p.splits);
+        zb = blockIdx.x / (2 * p.splits);
+    } else {
+        const uint32_t jb = blockIdx.x / 8;
+        pair = (jb / p.zs) * 8 + blockIdx.x % 8;
+        zb = jb % p.zs;
+        if (pair >= 2 * p.splits) return;   // padding of the grid to whole rounds of 8
+    }
+    const uint32_t split = pair >> 1, g = pair & 1, r0 = zb * kRowsPer;
     const uint32_t nr = min((uint32_t)kRowsPer, p.rows - r0);
     const uint32_t first_end = p.pos + r0 + 1, block_end = p.pos + r0 + nr;   // keys of the first and last row
     const uint32_t begin = split * p.split_chunks * kChunk;
@@ -1202,9 +1233,13 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
 
     // ---- the small loads first, then the first two chunks (as decode_int8_kernel)
     const uint32_t last = end - 1;
-    float ksv[kMaxSplitTokens / 512], vsv[kMaxSplitTokens / 512], vnew[kRowsPer];
+    // (the scales of a split of up to 512 tokens in one load each: the counts of further passes are
+    // uniform branches)
+    constexpr int kPasses = kMaxSplitTokens / 512;
+    float ksv[kPasses], vsv[kPasses], vnew[kRowsPer];
 #pragma unroll
-    for (int it = 0; it < kMaxSplitTokens / 512; it++) {
+    for (int it = 0; it < kPasses; it++) {
+        if (it > 0 && begin + 512 * it >= end) break;
         const size_t at = (size_t)min(begin + tid + 512 * it, last) * 2 + g;
         ksv[it] = p.ks[at];
         vsv[it] = p.vs[at];
@@ -1212,13 +1247,17 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     // the V scales of the tokens between the first and the last row's ends
 #pragma unroll
     for (int i = 0; i + 1 < kRowsPer; i++) vnew[i] = p.vs[(size_t)min(first_end + i, last) * 2 + g];
-    const int qct = CT == 2 ? wave >> 2 : 0, chunk = wave & 3;   // the query tile and step this wave builds
-    float4 x[4];
-    {
-        const uint32_t row = r0 + min((uint32_t)(2 * qct + (n >> 3)), nr - 1);
-        const float *qs = p.q + ((size_t)row * 16 + g * 8 + head) * 256 + 64 * chunk + 16 * qq;
+    // wave w builds the operands of head w of every row, lane holding dimensions 4 lane .. + 3
+    float4 x[kRowsPer];
 #pragma unroll
-        for (int f = 0; f < 4; f++) x[f] = *reinterpret_cast<const float4 *>(qs + 4 * f);
+    for (int r = 0; r < kRowsPer; r++) {
+        const uint32_t row = r0 + min((uint32_t)r, nr - 1);
+        if constexpr (kHalfQ) {   // exact in FP32
+            const half4 a = *reinterpret_cast<const half4 *>(p.qh + (((size_t)g * p.rows + row) * 8 + wave) * 256 + 4 * lane);
+            x[r] = make_float4((float)a[0], (float)a[1], (float)a[2], (float)a[3]);
+        } else {
+            x[r] = *reinterpret_cast<const float4 *>(p.q + ((size_t)row * 16 + g * 8 + wave) * 256 + 4 * lane);
+        }
     }
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
@@ -1271,24 +1310,55 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     load_k(kb, 1);
     load_v(vb, 1);
 
-    // ---- scales of the split into LDS, the columns' V scale references, the query's INT8 parts
-    float vmax = 0.0f;
+    // ---- the query's INT8 parts. z = q / s_q lies in [-127, 127]; q1 = rint(z), q2 = rint(254 r1) of
+    // the remainder r1 = z - q1 (|r1| <= 1/2) and q3 = rint(254 r2) of r2 = 254 r1 - q2. Adding 1.5 x
+    // 2^23 rounds to an integer whose low byte is its two's complement code: 7 operations an element
+    // where rint, clamp, convert and pack took 20 (8 waves on 4 SIMDs: 8 cycles each).
+    float amax[kRowsPer];
 #pragma unroll
-    for (int it = 0; it < kMaxSplitTokens / 512; it++) {
-        const uint32_t e = tid + 512 * it, t = begin + e;
-        kscale[e] = t < end ? ksv[it] * (kLog2e / 16.0f) : 0.0f;
-        vscale[e] = t < end ? vsv[it] : 0.0f;
-        vmax = fmaxf(vmax, t < min(end, first_end) ? vsv[it] : 0.0f);
+    for (int r = 0; r < kRowsPer; r++) amax[r] = fmaxf(fmaxf(fabsf(x[r].x), fabsf(x[r].y)), fmaxf(fabsf(x[r].z), fabsf(x[r].w)));
+    wave_allmax(amax);
+#pragma unroll
+    for (int r = 0; r < kRowsPer; r++) {
+        constexpr float kMagic = 12582912.0f;
+        const float inv = amax[r] > 0.0f ? 127.0f / amax[r] : 0.0f;
+        const float xs[4] = {x[r].x, x[r].y, x[r].z, x[r].w};
+        uint32_t t[3][4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float t1 = fmaf(xs[e], inv, kMagic), q1 = t1 - kMagic, r1 = fmaf(xs[e], inv, -q1);
+            const float t2 = fmaf(r1, 254.0f, kMagic), q2 = t2 - kMagic, r2 = fmaf(r1, 254.0f, -q2);
+            const float t3 = fmaf(r2, 254.0f, kMagic);
+            t[0][e] = __builtin_bit_cast(uint32_t, t1);
+            t[1][e] = __builtin_bit_cast(uint32_t, t2);
+            t[2][e] = __builtin_bit_cast(uint32_t, t3);
+        }
+        // dimension 4 lane: step c, block qq (of the operand's lanes), word lane % 4 of its 16 bytes
+        const int c = lane >> 4, bq = (lane >> 2) & 3, col = 8 * (r & 1) + wave;
+        const int slot = 16 * bq + (col ^ (4 * c + bq));
+#pragma unroll
+        for (int part = 0; part < 3; part++) {
+            const uint32_t lo = __builtin_amdgcn_perm(t[part][1], t[part][0], 0x0c0c0400u);
+            const uint32_t hi = __builtin_amdgcn_perm(t[part][3], t[part][2], 0x04000c0cu);
+            uint32_t *dst = reinterpret_cast<uint32_t *>(part < 2 ? &qlds[r >> 1][part][c][slot] : &q3lds[r >> 1][c][slot]);
+            dst[lane & 3] = lo | hi;
+        }
+        if (lane == 0) qmax[r >> 1][col] = amax[r];
     }
+    // ---- scales of the split into LDS, the work-group's largest V scale
+    float vmax[1] = {0.0f};
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
-    if (lane == 0) red[wave] = vmax;
-    float amax = 0.0f;
-#pragma unroll
-    for (int f = 0; f < 4; f++) amax = fmaxf(amax, fmaxf(fmaxf(fabsf(x[f].x), fabsf(x[f].y)), fmaxf(fabsf(x[f].z), fabsf(x[f].w))));
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-    if (lane < 16 && wave < 4 * CT) qmax[qct][chunk][lane] = amax;
+    for (int it = 0; it < kPasses; it++) {
+        if (it > 0 && begin + 512 * it >= end) break;
+        const uint32_t e = tid + 512 * it, t = begin + e;
+        kscale[e] = t < end ? ksv[it] * (kLog2e / 16.0f / 254.0f) : 0.0f;   // a dot's unit is 1 / 254 (below)
+        vscale[e] = t < end ? vsv[it] : 0.0f;
+        vmax[0] = fmaxf(vmax[0], t < min(end, first_end) ? vsv[it] : 0.0f);
+    }
+    wave_allmax(vmax);
+    if (lane == 0) red[wave] = vmax[0];
+    store_k(ka);
+    if (2 < nchunks) load_k(ka, 2);
     __syncthreads();
     // row i of the block sees the tokens before first_end and vnew[0 .. i - 1], where the split holds them
     float vcum = red[0];
@@ -1314,45 +1384,16 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         // its subnormals
         vinv[ct] = vref[ct] > 0.0f ? 128.0f / vref[ct] : 0.0f;
         vref[ct] *= 1.0f / 128.0f;
-        qsc[ct] = fmaxf(fmaxf(qmax[ct][0][n], qmax[ct][1][n]), fmaxf(qmax[ct][2][n], qmax[ct][3][n])) * (1.0f / 127.0f);
+        qsc[ct] = qmax[ct][n] * (1.0f / 127.0f);
         row_end[ct] = first_end + min((uint32_t)(2 * ct + (n >> 3)), nr - 1);
     }
-    {
-        const float qabs = fmaxf(fmaxf(qmax[qct][0][n], qmax[qct][1][n]), fmaxf(qmax[qct][2][n], qmax[qct][3][n]));
-        const float inv = qabs > 0.0f ? 127.0f / qabs : 0.0f;
-        auto code = [](float q) { return (uint32_t)(uint8_t)(int8_t)(int)fminf(fmaxf(q, -127.0f), 127.0f); };
-        uint32_t w1[4], w2[4], w3[4];
-#pragma unroll
-        for (int f = 0; f < 4; f++) {
-            const float xs[4] = {x[f].x, x[f].y, x[f].z, x[f].w};
-            w1[f] = w2[f] = w3[f] = 0;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {   // as decode_int8_kernel
-                const float z = xs[e] * inv, q1 = rintf(z), r1 = z - q1;
-                const float q2 = rintf(r1 * 254.0f);
-                const float r2 = fmaf(r1, 254.0f, -q2);
-                const float q3 = rintf(r2 * 254.0f);
-                w1[f] |= code(q1) << (8 * e);
-                w2[f] |= code(q2) << (8 * e);
-                w3[f] |= code(q3) << (8 * e);
-            }
-        }
-        if (wave < 4 * CT) {
-            qlds[qct][0][chunk][lane] = v4i{(int)w1[0], (int)w1[1], (int)w1[2], (int)w1[3]};
-            qlds[qct][1][chunk][lane] = v4i{(int)w2[0], (int)w2[1], (int)w2[2], (int)w2[3]};
-            q3lds[qct][chunk][lane] = v4i{(int)w3[0], (int)w3[1], (int)w3[2], (int)w3[3]};
-        }
-    }
-    store_k(ka);
-    if (2 < nchunks) load_k(ka, 2);
-    __syncthreads();
     v4i qi[CT][2][4];
 #pragma unroll
     for (int ct = 0; ct < CT; ct++)
 #pragma unroll
         for (int part = 0; part < 2; part++)
 #pragma unroll
-            for (int c = 0; c < 4; c++) qi[ct][part][c] = qlds[ct][part][c][lane];
+            for (int c = 0; c < 4; c++) qi[ct][part][c] = qlds[ct][part][c][16 * qq + (n ^ (4 * c + qq))];
 
     floatx4 o[2][CT];   // O^T: dimensions 32 wave + 16 dt + 4 qq + r of column n
     float m[CT], l[CT], total_prev[CT], dot_prev[CT][4];   // l: this lane's tokens, summed over lanes at the end
@@ -1364,34 +1405,43 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
 #pragma unroll
         for (int r = 0; r < 4; r++) dot_prev[ct][r] = 0.0f;
     }
-    int local_prev = 0;
-    auto probs = [&](int slot) __attribute__((always_inline)) {
-        const float4 vs4 = *reinterpret_cast<const float4 *>(&vscale[local_prev]);
-        const float4 ks4 = *reinterpret_cast<const float4 *>(&kscale[local_prev]);
+    auto probs = [&](uint32_t j) __attribute__((always_inline)) {
+        const int slot = j & 1, local0 = (int)(j * kChunk) + 16 * wave + 4 * qq;
+        const float4 vs4 = *reinterpret_cast<const float4 *>(&vscale[local0]);
+        const float4 ks4 = *reinterpret_cast<const float4 *>(&kscale[local0]);
         const float vsr[4] = {vs4.x, vs4.y, vs4.z, vs4.w}, ksr[4] = {ks4.x, ks4.y, ks4.z, ks4.w};
-        const uint32_t t0 = begin + (uint32_t)local_prev;
+        const uint32_t t0 = begin + (uint32_t)local0;
+        const bool edge = begin + (j + 1) * kChunk > first_end;   // some row does not see the whole chunk
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) {
-            // m = -inf (before the column's first rescale): its operands are rebuilt before they are read
+            // m = -inf only in a column without a score yet
             const float refc = fmaxf(m[ct], -3.0e38f);
-            half4 hi, lo;
+            float arg[4], scaled[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) arg[r] = fmaf(dot_prev[ct][r], qsc[ct] * ksr[r], -refc);
+            if (edge)   // uniform
+#pragma unroll
+                for (int r = 0; r < 4; r++) arg[r] = t0 + r < row_end[ct] ? arg[r] : -INFINITY;
             float total = 0.0f;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float arg = fmaf(dot_prev[ct][r], qsc[ct] * ksr[r], -refc);
-                const float prob = __builtin_amdgcn_exp2f(t0 + r < row_end[ct] ? arg : -INFINITY);
+                const float prob = __builtin_amdgcn_exp2f(arg[r]);   // 0 for masked tokens
                 total += prob;
-                float scaled = prob * (vsr[r] * vinv[ct]);
+                scaled[r] = prob * (vsr[r] * vinv[ct]);
                 // one rounded FP32 value: else the operand's hi is the exact product rounded once
                 // (v_fma_mixlo_f16) and the hi that lo completes the rounded product rounded again,
                 // which differ by 2^-10 in rare near-ties
-                asm("" : "+v"(scaled));
-                hi[r] = (_Float16)scaled;
-                lo[r] = (_Float16)(scaled - (float)hi[r]);
+                asm("" : "+v"(scaled[r]));
             }
             total_prev[ct] = total;
-            pshare[slot][ct][0][wave][lane] = __builtin_bit_cast(uint2, hi);
-            pshare[slot][ct][1][wave][lane] = __builtin_bit_cast(uint2, lo);
+            half4 hi, lo;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                hi[r] = (_Float16)scaled[r];
+                lo[r] = (_Float16)(scaled[r] - (float)hi[r]);
+            }
+            pshare[slot][ct][0][wave][n][qq] = __builtin_bit_cast(uint2, hi);
+            pshare[slot][ct][1][wave][n][qq] = __builtin_bit_cast(uint2, lo);
         }
     };
     // the phases of decode_int8_kernel: finish chunk j - 1, score chunk j, stage V of chunk j and K of
@@ -1402,14 +1452,15 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         bool raise = false;
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) {
-            ctop[ct] = chunk_top[slot][ct][0][n];
-#pragma unroll
-            for (int w = 1; w < kDecodeWaves; w++) ctop[ct] = fmaxf(ctop[ct], chunk_top[slot][ct][w][n]);
+            const float4 a = *reinterpret_cast<const float4 *>(&chunk_top[slot][ct][n][0]);
+            const float4 b = *reinterpret_cast<const float4 *>(&chunk_top[slot][ct][n][4]);
+            ctop[ct] = fmaxf(fmaxf(fmaxf(a.x, a.y), fmaxf(a.z, a.w)), fmaxf(fmaxf(b.x, b.y), fmaxf(b.z, b.w)));
             raise |= ctop[ct] > m[ct] + 8.0f;
         }
         // every wave reads the same maxima: the branch is uniform over the work-group. Only the
-        // columns that passed the bound change (the others' factor is 1 and their operands the same)
-        if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+        // columns that passed the bound change (the others' factor is 1 and their operands the same).
+        // Chunk 0 has no reference before its maxima: its operands are made here
+        if (j == 1 || __builtin_amdgcn_ballot_w64(raise) != 0) {
 #pragma unroll
             for (int ct = 0; ct < CT; ct++) {
                 const float next = ctop[ct] > m[ct] + 8.0f ? ctop[ct] : m[ct];
@@ -1419,22 +1470,20 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
                 o[1][ct] *= decay;
                 m[ct] = next;
             }
-            probs(slot);
+            probs(j - 1);
             __syncthreads();
         }
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) l[ct] += total_prev[ct];
 #pragma unroll
         for (int s = 0; s < kDecodeWaves / 2; s++) {
-            const int src = 2 * s + (qq >> 1), at = n + 32 * (qq & 1);
+            const int src = 2 * s + (qq >> 1);
             half8 ps[CT][2];
 #pragma unroll
             for (int ct = 0; ct < CT; ct++)
 #pragma unroll
-                for (int hl = 0; hl < 2; hl++) {
-                    const uint2 pa = pshare[slot][ct][hl][src][at], pb = pshare[slot][ct][hl][src][at + 16];
-                    ps[ct][hl] = __builtin_bit_cast(half8, make_uint4(pa.x, pa.y, pb.x, pb.y));
-                }
+                for (int hl = 0; hl < 2; hl++)
+                    ps[ct][hl] = *reinterpret_cast<const half8 *>(&pshare[slot][ct][hl][src][n][2 * (qq & 1)]);
 #pragma unroll
             for (int dt = 0; dt < 2; dt++) {
                 const int d = 16 * (2 * wave + dt) + n;
@@ -1463,36 +1512,50 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
 #pragma unroll
             for (int jj = 0; jj < 4; jj++) {
                 const v4i kop = __builtin_bit_cast(v4i, kbuf[wave][n][(4 * jj + qq) ^ n]);
+                const int slot = 16 * qq + (n ^ (4 * jj + qq));
 #pragma unroll
                 for (int ct = 0; ct < CT; ct++) {
                     acc[ct][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, qi[ct][0][jj], acc[ct][0], 0, 0, 0);
                     acc[ct][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, qi[ct][1][jj], acc[ct][1], 0, 0, 0);
-                    acc[ct][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, q3lds[ct][jj][lane], acc[ct][2], 0, 0, 0);
+                    acc[ct][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, q3lds[ct][jj][slot], acc[ct][2], 0, 0, 0);
                 }
             }
             const int local0 = (int)(j * kChunk) + 16 * wave + 4 * qq;   // token offset inside the split
             const uint32_t t0 = begin + (uint32_t)local0;
+            const bool edge = begin + (j + 1) * kChunk > first_end;
             const float4 ks4 = *reinterpret_cast<const float4 *>(&kscale[local0]);
             const float ksr[4] = {ks4.x, ks4.y, ks4.z, ks4.w};
-            local_prev = local0;
+            float top[CT];
 #pragma unroll
             for (int ct = 0; ct < CT; ct++) {
-                float top = -INFINITY;
+                float score[4];
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    // every dot is an integer below 2^22 in magnitude, exact in FP32. The exponent's
-                    // argument is one fma of the dot (probs), so the score itself, rounded, is only
-                    // compared
-                    const float full = fmaf((float)acc[ct][2][r], 1.0f / 64516.0f,
-                                            fmaf((float)acc[ct][1][r], 1.0f / 254.0f, (float)acc[ct][0][r]));
-                    dot_prev[ct][r] = full;
-                    top = fmaxf(top, t0 + r < row_end[ct] ? full * (qsc[ct] * ksr[r]) : -INFINITY);
+                    // 254 dot1 + dot2 is an exact integer (|dots| < 2^22) and the dot's unit 1 / 254. The
+                    // exponent's argument is one fma of the dot (probs), so the score itself, rounded,
+                    // is only compared
+                    const float d12 = (float)(__mul24(acc[ct][0][r], 254) + acc[ct][1][r]);
+                    dot_prev[ct][r] = fmaf((float)acc[ct][2][r], 1.0f / 254.0f, d12);
+                    score[r] = dot_prev[ct][r] * (qsc[ct] * ksr[r]);
                 }
-                top = xl_max16(top);
-                top = xl_max32(top);
-                if (qq == 0) chunk_top[j & 1][ct][wave][n] = top;
+                if (edge)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) score[r] = t0 + r < row_end[ct] ? score[r] : -INFINITY;
+                top[ct] = fmaxf(fmaxf(score[0], score[1]), fmaxf(score[2], score[3]));
             }
-            probs(j & 1);
+            // over the lanes of a column: with two tiles one swap of halves serves both, lanes below 32
+            // ending with tile 0's maximum and the others with tile 1's
+            float t = top[0];
+            if constexpr (CT == 2) {
+                float u = top[1];
+                asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(t), "+v"(u));
+                t = fmaxf(t, u);
+            } else {
+                t = xl_max32(t);
+            }
+            t = xl_max16(t);
+            if ((qq & 1) == 0 && (CT == 2 || qq == 0)) chunk_top[j & 1][CT == 2 ? qq >> 1 : 0][n][wave] = t;
+            if (j > 0) probs(j);
         }
         store_v(j & 1, rv);
         if (load_v2) load_v(rv, j + 2);
@@ -1521,44 +1584,65 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     }
     finish(last_phase);
 
-    // ---- l over the lanes and waves; O^T[d][n] times the column's V scale reference
+    // ---- O^T[d][n] times the column's V scale reference, l over the lanes and waves
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) {
         const float lt = xl_sum32(xl_sum16(l[ct]));
         if (qq == 0) wave_l[ct][wave][n] = lt;
     }
+    if (p.splits > 1) {   // the partials' O needs no other wave's l
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+            const uint32_t ri = 2 * ct + (n >> 3);
+            if (ri >= nr) continue;
+            float *part = part_of(ri) + head * 256 + 32 * wave + 4 * qq;
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++)
+                *reinterpret_cast<float4 *>(part + 16 * dt) = make_float4(o[dt][ct][0] * vref[ct], o[dt][ct][1] * vref[ct],
+                                                                          o[dt][ct][2] * vref[ct], o[dt][ct][3] * vref[ct]);
+        }
+        __syncthreads();
+        if (wave == 0 && qq == 0) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++) {
+                const uint32_t ri = 2 * ct + (n >> 3);
+                if (ri >= nr) continue;
+                float lw = 0.0f;
+#pragma unroll
+                for (int w = 0; w < kDecodeWaves; w++) lw += wave_l[ct][w][n];
+                float *part = part_of(ri);
+                part[2048 + head] = m[ct];
+                part[2056 + head] = lw;
+            }
+        }
+        return;
+    }
+    // gate and y need only 4-byte alignment; all gate loads go out before the first store (the
+    // compiler cannot tell y from gate)
+    float gate[CT][2][4];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        const uint32_t row = r0 + min((uint32_t)(2 * ct + (n >> 3)), nr - 1);
+        const float *at = p.gate + ((size_t)row * 16 + g * 8 + head) * 256 + 32 * wave + 4 * qq;
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) gate[ct][dt][e] = at[16 * dt + e];
+    }
     __syncthreads();
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) {
         const uint32_t ri = 2 * ct + (n >> 3);
-        if (ri >= nr) continue;
         float lw = 0.0f;
 #pragma unroll
         for (int w = 0; w < kDecodeWaves; w++) lw += wave_l[ct][w][n];
-        if (p.splits == 1) {
-            const float inv = 1.0f / lw;
-#pragma unroll
-            for (int dt = 0; dt < 2; dt++) {
-                // gate and y need only 4-byte alignment (the gate loads go out before the first store)
-                const size_t at = ((size_t)(r0 + ri) * 16 + g * 8 + head) * 256 + 32 * wave + 16 * dt + 4 * qq;
-                const float g0 = p.gate[at + 0], g1 = p.gate[at + 1], g2 = p.gate[at + 2], g3 = p.gate[at + 3];
-                asm volatile("" ::"v"(g0), "v"(g1), "v"(g2), "v"(g3) : "memory");
-                p.y[at + 0] = o[dt][ct][0] * vref[ct] * inv * sigmoidf(g0);
-                p.y[at + 1] = o[dt][ct][1] * vref[ct] * inv * sigmoidf(g1);
-                p.y[at + 2] = o[dt][ct][2] * vref[ct] * inv * sigmoidf(g2);
-                p.y[at + 3] = o[dt][ct][3] * vref[ct] * inv * sigmoidf(g3);
-            }
-            continue;
-        }
-        float *part = part_of(ri);
+        if (ri >= nr) continue;
+        const float inv = 1.0f / lw;
+        float *at = p.y + ((size_t)(r0 + ri) * 16 + g * 8 + head) * 256 + 32 * wave + 4 * qq;
 #pragma unroll
         for (int dt = 0; dt < 2; dt++)
-            *reinterpret_cast<float4 *>(part + head * 256 + 32 * wave + 16 * dt + 4 * qq) =
-                make_float4(o[dt][ct][0] * vref[ct], o[dt][ct][1] * vref[ct], o[dt][ct][2] * vref[ct], o[dt][ct][3] * vref[ct]);
-        if (wave == 0 && qq == 0) {
-            part[2048 + head] = m[ct];
-            part[2056 + head] = lw;
-        }
+#pragma unroll
+            for (int e = 0; e < 4; e++) at[16 * dt + e] = o[dt][ct][e] * vref[ct] * inv * sigmoidf(gate[ct][dt][e]);
     }
 }
 
@@ -1815,6 +1899,7 @@ const char *launch_verify_int8(Context &c, const View *b, int count, const boot_
         uint64_t next = first + 1;
         while (next < rows && split_of(next) == split_of(first)) next++;
         RowsParams d;
+        d.qh = nullptr;
         d.q = (const float *)b[0].ptr + first * 4096;
         d.k = (const int8_t *)b[1].ptr;
         d.v = (const int8_t *)b[2].ptr;
@@ -1836,7 +1921,9 @@ const char *launch_verify_int8(Context &c, const View *b, int count, const boot_
         d.zs = narrow ? 1 : (d.rows + 3) / 4;
         const dim3 grid((2 * d.splits + 7) / 8 * 8 * d.zs);
         launch_timed(c, "rows_int8_kernel",
-                     narrow ? rows_int8_kernel<1, true> : d.zs == 1 ? rows_int8_kernel<2, true> : rows_int8_kernel<2, false>,
+                     narrow        ? rows_int8_kernel<1, true, false>
+                     : d.zs == 1 ? rows_int8_kernel<2, true, false>
+                                 : rows_int8_kernel<2, false, false>,
                      grid, dim3(512), d);
         if (d.splits > 1)
             launch_timed(c, "decode_combine_kernel", decode_combine_kernel, dim3(4, 16, d.rows), dim3(256),
@@ -1870,6 +1957,47 @@ const char *launch_online_int8_as_decode(Context &c, const View *b, const boot_k
     d.k_out = d.v_out = nullptr;
     d.ks_out = d.vs_out = nullptr;
     return decode_launch<true>(c, d, rows, length);
+}
+
+const char *launch_online_int8_rows(Context &c, const View *b, const boot_kernel_args &p) {
+    // A prefill chunk on rows_int8_kernel (launch_prefill's choice, which has validated the bindings:
+    // grouped FP16 q, k, v, gate, y, ks, vs).
+    const uint64_t rows = p.m, length = (uint64_t)p.pos + rows;
+    BOOT_REQUIRE(rows >= 1 && rows <= 512, "a prefill chunk served by the multi-row kernel has 1 to 512 rows");
+    RowsParams d;
+    d.q = nullptr;
+    d.qh = (const _Float16 *)b[0].ptr;
+    d.k = (const int8_t *)b[1].ptr;
+    d.v = (const int8_t *)b[2].ptr;
+    d.gate = (const float *)b[3].ptr;
+    d.y = (float *)b[4].ptr;
+    d.ks = (const float *)b[5].ptr;
+    d.vs = (const float *)b[6].ptr;
+    d.rows = (uint32_t)rows;
+    d.pos = p.pos;
+    d.zs = (uint32_t)((rows + 3) / 4);
+    // One split, or one round of work-groups: a chunk of 128 keys takes about 2.4 us of a work-group,
+    // the combine 4 us and 0.067 us per row (64 rows after 200 keys: 3 splits 18.0, one 15.2 us; 8
+    // rows after 1000: 8 splits 14.0 us, one about 27). More than 64 rows are never split (the
+    // combine of 200 rows takes 21 us).
+    const uint64_t chunks = (length + kChunk - 1) / kChunk;
+    const uint64_t slots = rows > 64 ? 1 : std::max<uint64_t>(1, (uint64_t)std::max(1, context_cus(c)) / (2 * d.zs));
+    const uint64_t most = kMaxSplitTokens / kChunk, spread = std::min<uint64_t>((chunks + slots - 1) / slots, most);
+    const uint64_t split_chunks = 24 * (chunks - spread) <= 40 + 2 * rows / 3 && chunks <= most ? chunks : spread;
+    d.split_chunks = (uint32_t)split_chunks;
+    d.splits = (uint32_t)((chunks + split_chunks - 1) / split_chunks);
+    d.partial = nullptr;
+    if (d.splits > 1) {
+        d.partial = (float *)context_workspace(c, rows * 2 * d.splits * kPartialFloats * sizeof(float));
+        BOOT_REQUIRE(d.partial, "cannot allocate prefill split workspace");
+    }
+    launch_timed(c, "rows_int8_half_query_kernel", rows_int8_kernel<2, false, true>, dim3(2 * d.splits * d.zs), dim3(512), d);
+    if (d.splits > 1) {
+        context_split(c, "attention_online_int8.combine");
+        launch_timed(c, "decode_combine_kernel", decode_combine_kernel, dim3(4, 16, d.rows), dim3(256),
+                     (const float *)d.partial, d.gate, d.y, d.splits);
+    }
+    return nullptr;
 }
 
 }  // namespace boot

@@ -57,8 +57,9 @@ constexpr size_t kPartialBytes = 2 * kPartialRegion + 3 * kTileRows * 4;
 // A row's partial is FP16 when its outputs are at most this large (FP16's relative 2^-12 of 4 is
 // 9.8e-4), FP32 otherwise.
 constexpr float kNarrowPartial = 4.0f;
-// Prefill chunks of at most 64 rows with rows x keys up to this go through the decode kernel.
-constexpr uint64_t kDecodeRouteWork = 65536;
+// Few rows with rows x keys up to these go through the decode kernel (16 rows) and the multi-row
+// kernel (64 rows); see launch_prefill.
+constexpr uint64_t kDecodeRouteWork = 32768, kRowsRouteWork = 524288;
 
 struct PrefillParams {
     const _Float16 *q;      // grouped FP16 [2][M][8][256]
@@ -1163,11 +1164,22 @@ const char *launch_prefill(Context &c, const View *b, const boot_kernel_args &a,
     BOOT_REQUIRE(aligned(b[0].ptr, 16) && aligned(b[1].ptr, 16) && aligned(b[2].ptr, 16) && aligned(b[3].ptr, 16) &&
                      aligned(b[4].ptr, 16),
                  "bindings misaligned (q, k, v, gate, y need 16 bytes)");
-    // Chunks of at most 64 rows whose rows x keys stay within kDecodeRouteWork go to the decode
-    // kernel (one work-group per row, KV group and split of the keys): at (0, 33) 7.6 against
-    // 25.4 us, at (2048, 33) 24.8 against 38.4 us; each row reads the keys again, so at (8192, 33)
-    // it would take 81 against 44 us.
-    if (int8 && rows <= 64 && rows * keys <= kDecodeRouteWork) return launch_online_int8_as_decode(c, b, a);
+    // Small work does not fill this kernel's 256-row tiles, and its launch costs about 17 us beyond its
+    // key tiles, plus a combine. Attention + combine, one box, decode kernel / multi-row kernel / this:
+    // * one chunk of 128 keys, or few rows over little history: the decode kernel, one work-group per
+    //   row, KV group and split: (0, 64) 8.1 / 11.2 / 20.8, (1000, 16) 14.0 / 14.8 / 21.3, (2000, 8)
+    //   13.6 / 15.3 / 22.8; (500, 33) 16.4 / 16.1, (1000, 64) 24.6 / 21.8 us;
+    // * up to 64 rows and 2^19 row-key pairs: the multi-row kernel, which reads the keys once per four
+    //   rows: (8000, 16) 26.7 / 20.9 / 41.0, (30000, 12) - / 29.2 / 50.9, (12000, 40) - / 38.2 / 40.9,
+    //   (8000, 64) - / 39.7 / 39.3 us;
+    // * up to 512 rows in one split, 8 us and 2.4 us per 128 keys: (0, 256) 13.6 / 24.2, (600, 400)
+    //   28.7 / 35.5, (700, 200) 27.0 / 30.9, (1100, 256) 34.4 / 33.3, (1024, 512) 39.8 / 38.9 us.
+    if (int8 && rows <= 512) {
+        const uint64_t chunks = (keys + 127) / 128, work = rows * keys;
+        if (rows <= 64 && (chunks == 1 || (rows <= 16 && work <= kDecodeRouteWork)))
+            return launch_online_int8_as_decode(c, b, a);
+        if (rows <= 64 ? work <= kRowsRouteWork : 80 * chunks <= 520 + rows) return launch_online_int8_rows(c, b, a);
+    }
     PrefillParams p;
     p.q = (const _Float16 *)b[0].ptr;
     p.k = b[1].ptr;
@@ -1193,6 +1205,7 @@ const char *launch_prefill(Context &c, const View *b, const boot_kernel_args &a,
     const uint64_t base_blocks = 2ull * p.tiles;
     const uint64_t round = (uint64_t)std::max(1, context_cus(c));
     uint64_t splits = std::max<uint64_t>(1, std::min<uint64_t>(round / base_blocks, keys / kW64Keys));
+    if (keys < 512) splits = 1;   // (FP16 storage only) few keys: the partials' FP16 rounding would show
     uint64_t split_keys = (keys + splits - 1) / splits;
     split_keys = (split_keys + kW64Keys - 1) / kW64Keys * kW64Keys;
     splits = (keys + split_keys - 1) / split_keys;

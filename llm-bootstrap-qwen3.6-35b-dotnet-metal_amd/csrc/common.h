@@ -90,6 +90,9 @@ const char *launch_decode_int8(Context &, const View *, int, const boot_kernel_a
 // attention_online_int8 for chunks of at most 64 rows over a short history, through the decode
 // kernel (bindings validated by the prefill launcher)
 const char *launch_online_int8_as_decode(Context &, const View *, const boot_kernel_args &);
+// and for chunks of at most 512 rows over up to about 1500 keys, or of few rows over longer ones,
+// through the multi-row kernel
+const char *launch_online_int8_rows(Context &, const View *, const boot_kernel_args &);
 const char *launch_decode_append_int8(Context &, const View *, int, const boot_kernel_args &, const uint32_t *);
 const char *launch_verify_int8(Context &, const View *, int, const boot_kernel_args &, const uint32_t *);
 const char *launch_scores_int8(Context &, const View *, int, const boot_kernel_args &, const uint32_t *);

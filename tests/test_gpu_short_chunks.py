@@ -1,5 +1,7 @@
-"""Prefill chunks over short key ranges: one or two 32-key tiles per split, the last one ragged,
-and row tiles whose causal end lies splits before the range's end."""
+"""Prefill chunks over short key ranges and of few rows: the multi-row kernel (whole and partial row
+blocks, row blocks whose causal end lies chunks or splits before the range's end, one split and
+several), its edges against the decode kernel and the 256-row kernel, and that kernel's splits of one
+or two 32-key tiles, the last one ragged."""
 import numpy as np
 import pytest
 
@@ -9,10 +11,15 @@ from test_gpu_attention import MAX_ABS, REL_L2, build_case, run_prefill
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("history,rows", [(0, 65), (0, 96), (0, 97), (7, 120), (0, 255), (31, 257), (500, 480), (993, 513)])
+@pytest.mark.parametrize("history,rows", [
+    (0, 65), (0, 97), (7, 120), (0, 255), (31, 257), (500, 480), (1023, 512),      # multi-row, one split
+    (112, 17), (1000, 33), (2031, 17), (8128, 64), (4000, 8), (60000, 5),          # multi-row, few rows
+    (64, 64), (112, 16), (2000, 16), (2033, 16),                                   # around the decode kernel
+    (801, 100), (1025, 512), (993, 513), (0, 600)])                                # 256-row kernel
 def test_prefill_short_ranges(device, oracle, history, rows):
     """Against FP64 at the bounds of the other prefill tests: rel-L2 1e-3, max-abs 2e-3 and the
-    reference's per-element bound (FP16 operands and FP16 split partials, 2^-12 relative each)."""
+    reference's per-element bound (the 256-row kernel's FP16 operands and partials, 2^-12 relative
+    each; the others are FP32-accurate)."""
     q, gate, host = build_case(oracle, history, rows)
     cache = upload_cache(device, *host)
     y = run_prefill(device, q, gate, cache, rows, history)
