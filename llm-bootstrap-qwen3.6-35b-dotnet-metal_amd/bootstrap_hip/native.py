@@ -12,7 +12,9 @@ There is no CPU fallback: if the library or a gfx950 device is missing, construc
 from __future__ import annotations
 
 import ctypes
+import operator
 import os
+import struct
 import weakref
 from typing import NamedTuple, Optional
 
@@ -49,9 +51,10 @@ SIGNATURES = {
     "boot_allocated": (_U64, [_VP]),
     "boot_begin": (_I, [_VP]),
     "boot_clear": (_I, [_VP, _VP]),
-    "boot_dispatch": (_I, [_VP, _CP, ctypes.POINTER(_VP), ctypes.POINTER(_U64), _I, _VP, _I,
+    # (the handle and offset arrays as plain pointers: ctypes arrays or packed bytes)
+    "boot_dispatch": (_I, [_VP, _CP, _VP, _VP, _I, _VP, _I,
                            _U32, _U32, _U32, _U32, _U32, _U32, _VP, _U64]),
-    "boot_dispatch_noalloc": (_I, [_VP, _CP, ctypes.POINTER(_VP), ctypes.POINTER(_U64), _I, _VP, _I,
+    "boot_dispatch_noalloc": (_I, [_VP, _CP, _VP, _VP, _I, _VP, _I,
                                    _U32, _U32, _U32, _U32, _U32, _U32, _VP, _U64]),
     "boot_end": (_I, [_VP]),
     "boot_profile": (None, [_VP, _I]),
@@ -63,6 +66,12 @@ SIGNATURES = {
     "boot_write": (_I, [_VP, _VP, _U64, _VP, _U64]),
     "boot_read": (_I, [_VP, _VP, _U64, _VP, _U64]),
 }
+
+# Packers of n handles or offsets: one call each, where filling a ctypes array converts element by
+# element
+_PACKERS = tuple(struct.Struct(f"{n}Q").pack for n in range(32))
+_ARGS_BYTES = ctypes.sizeof(KernelArgs)
+_byref, _NO_OFFSET = ctypes.byref, ctypes.c_uint64(0)
 
 _lib: Optional[ctypes.CDLL] = None
 
@@ -149,6 +158,10 @@ class Device:
         if not handle:
             raise HipError("HIP device unavailable or not gfx950 (boot_create returned NULL)")
         self.handle = handle
+        self._context = ctypes.c_void_p(handle)
+        # boot_dispatch, boot_dispatch_noalloc as their own function objects: converting fifteen
+        # arguments by declared types costs 1.5 us a call
+        self._entries = (self.lib["boot_dispatch"], self.lib["boot_dispatch_noalloc"])
         self._live = weakref.WeakSet()   # buffers whose handles close() must invalidate
 
     # Metal.cs:69
@@ -209,23 +222,42 @@ class Device:
     def dispatch(self, kernel: str, args: KernelArgs, threads: int, group: int, *bindings,
                  noalloc: bool = False) -> None:
         """Metal.cs:96-97."""
-        self.dispatch2d(kernel, args, threads, 1, group, *bindings, noalloc=noalloc)
+        self._dispatch(kernel, args, threads, 1, group, bindings, noalloc)
 
     def dispatch2d(self, kernel: str, args: KernelArgs, threads_x: int, threads_y: int, group: int,
                    *bindings, noalloc: bool = False) -> None:
         """Metal.cs:98-104. ``noalloc`` routes through boot_dispatch_noalloc (split-K scratch
         from the library's static device array; no allocation, no timing sample)."""
+        self._dispatch(kernel, args, threads_x, threads_y, group, bindings, noalloc)
+
+    def _dispatch(self, kernel, args, threads_x, threads_y, group, bindings, noalloc) -> None:
         count = len(bindings)
-        handles = (ctypes.c_void_p * max(count, 1))()
-        offsets = (ctypes.c_uint64 * max(count, 1))()
-        for i, b in enumerate(bindings):
-            if isinstance(b, GpuBuffer):
-                b = Binding(b, 0)
-            handles[i] = b.buffer.handle
-            offsets[i] = b.offset
-        entry = self.lib.boot_dispatch_noalloc if noalloc else self.lib.boot_dispatch
-        self._check(entry(self.handle, kernel.encode(), handles, offsets, count, ctypes.byref(args),
-                          ctypes.sizeof(KernelArgs), threads_x, threads_y, 1, group, 1, 1, None, 0))
+        handles = [b.handle for b in bindings if isinstance(b, GpuBuffer)]
+        if len(handles) == count:
+            offsets = None   # all zero
+        else:
+            handles, offsets = [], []
+            for b in bindings:
+                if isinstance(b, GpuBuffer):
+                    handles.append(b.handle)
+                    offsets.append(0)
+                else:
+                    handles.append(b.buffer.handle)
+                    offsets.append(b.offset)
+        try:
+            pack = _PACKERS[count]
+            handles = pack(*handles)
+            if offsets is not None:
+                offsets = pack(*offsets)
+        except (struct.error, IndexError):   # more bindings; offsets outside 64 bits wrap as in C
+            pack = struct.Struct(f"{count}Q").pack
+            handles = handles if isinstance(handles, bytes) else pack(*handles)
+            if offsets is not None:
+                offsets = pack(*[operator.index(v) & 0xFFFFFFFFFFFFFFFF for v in offsets])
+        # (called without argument types: every argument is already the C type it is passed as)
+        if self._entries[noalloc](self._context, kernel.encode(), handles, offsets, count, _byref(args), _ARGS_BYTES,
+                                  threads_x, threads_y, 1, group, 1, 1, None, _NO_OFFSET) == 0:
+            self._check(0)
 
     def close(self) -> None:
         """Metal.cs:114. boot_destroy frees the context and every buffer it still owns, so the
@@ -236,6 +268,7 @@ class Device:
             self._live.clear()
             self.lib.boot_destroy(self.handle)
             self.handle = 0
+            self._context = None
 
     def __enter__(self):
         return self

@@ -1823,7 +1823,7 @@ const char *launch_decode_append_int8(Context &c, const View *b, int count, cons
     d.y = (float *)b[9].ptr;
     d.pos = p.pos;
     d.append = 1;
-    d.freq = rope_frequencies(p.theta);
+    d.freq = context_rope(c, p.theta);
     return decode_launch(c, d, 1, length);
 }
 

@@ -389,7 +389,7 @@ const char *launch_batch_rope_int8(Context &c, const View *b, int count, const b
     launch_timed(c, "batch_rope_int8_kernel", batch_rope_int8_kernel, dim3(blocks), dim3(256), 
         (const float *)b[0].ptr, (const float *)b[1].ptr, (const float *)b[2].ptr, (float *)b[3].ptr,
         (int8_t *)b[4].ptr, (int8_t *)b[5].ptr, (float *)b[6].ptr, (float *)b[7].ptr, (uint32_t)rows,
-        p.pos, rope_frequencies(p.theta), qblocks, first);
+        p.pos, context_rope(c, p.theta), qblocks, first);
     return nullptr;
 }
 
@@ -429,7 +429,7 @@ const char *launch_prepare_fused_int8(Context &c, const View *b, int count, cons
     launch_timed(c, "prepare_fused_int8_kernel", prepare_fused_int8_kernel, dim3(qblocks + (last - first + 1) * 2), dim3(256), 
         (const float *)b[0].ptr, (const float *)b[1].ptr, (const float *)b[2].ptr, (const uint16_t *)b[3].ptr,
         (const uint16_t *)b[4].ptr, (_Float16 *)b[5].ptr, (float *)b[6].ptr, (int8_t *)b[7].ptr, (int8_t *)b[8].ptr,
-        (float *)b[9].ptr, (float *)b[10].ptr, (uint32_t)rows, p.pos, rope_frequencies(p.theta), p.eps, qblocks, first);
+        (float *)b[9].ptr, (float *)b[10].ptr, (uint32_t)rows, p.pos, context_rope(c, p.theta), p.eps, qblocks, first);
     return nullptr;
 }
 
@@ -452,7 +452,7 @@ const char *launch_prepare_fused_half(Context &c, const View *b, int count, cons
     launch_timed(c, "prepare_fused_half_kernel", prepare_fused_half_kernel, dim3((uint32_t)(rows + (rows + 3) / 4)), dim3(256),
         (const float *)b[0].ptr, (const float *)b[1].ptr, (const float *)b[2].ptr, (const uint16_t *)b[3].ptr,
         (const uint16_t *)b[4].ptr, (_Float16 *)b[5].ptr, (float *)b[6].ptr, (_Float16 *)b[7].ptr,
-        (_Float16 *)b[8].ptr, (uint32_t)rows, p.pos, rope_frequencies(p.theta), p.eps);
+        (_Float16 *)b[8].ptr, (uint32_t)rows, p.pos, context_rope(c, p.theta), p.eps);
     return nullptr;
 }
 
@@ -470,7 +470,7 @@ const char *launch_batch_rope_half(Context &c, const View *b, int count, const b
                  "bindings misaligned");
     launch_timed(c, "batch_rope_half_kernel", batch_rope_half_kernel, dim3((uint32_t)((rows + 3) / 4)), dim3(256), 
         (const float *)b[0].ptr, (const float *)b[1].ptr, (const float *)b[2].ptr, (float *)b[3].ptr,
-        (_Float16 *)b[4].ptr, (_Float16 *)b[5].ptr, (uint32_t)rows, p.pos, rope_frequencies(p.theta));
+        (_Float16 *)b[4].ptr, (_Float16 *)b[5].ptr, (uint32_t)rows, p.pos, context_rope(c, p.theta));
     return nullptr;
 }
 

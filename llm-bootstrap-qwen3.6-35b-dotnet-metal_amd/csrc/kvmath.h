@@ -86,6 +86,11 @@ __host__ inline RopeFreq rope_frequencies(float theta) {
     return t;
 }
 
+// rope_frequencies(theta), evaluated anew only when theta changes: a model has one theta, and the 32
+// FP64 powers cost a dispatch 1 us of host time.
+struct Context;
+const RopeFreq &context_rope(Context &c, float theta);
+
 // Lane j < 32 of the wave gets frequency j (selected from the kernel argument's scalar values,
 // no memory access per lane); lanes 32..63 get 0.
 __device__ inline float lane_inv_freq(const RopeFreq &t) {

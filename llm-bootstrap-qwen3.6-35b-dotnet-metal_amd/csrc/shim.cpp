@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "common.h"
+#include "kvmath.h"
 
 namespace boot {
 
@@ -115,6 +116,10 @@ struct Context {
     std::string current_name;
     hipEvent_t current_start = nullptr;
     int current_kind = -1;
+    // context_rope: the frequencies of the last theta
+    uint32_t rope_theta = 0;
+    bool rope_valid = false;
+    RopeFreq rope;
 };
 
 namespace {
@@ -155,33 +160,32 @@ hipEvent_t record(Context *c) {
 }
 
 struct Entry {
+    const char *name;
     Launcher launch;
     int kind;  // attention sample kind: 0 QK, 1 softmax, 2 AV, 3 fused online/decode, -1 other
 };
 
-const std::unordered_map<std::string, Entry> &registry() {
-    static const std::unordered_map<std::string, Entry> table = {
-        {"kv_store_int8", {launch_kv_store_int8, -1}},
-        {"batch_rope_int8", {launch_batch_rope_int8, -1}},
-        {"attention_query_grouped_half", {launch_query_grouped_half, -1}},
-        {"attention_prepare_fused_int8", {launch_prepare_fused_int8, -1}},
-        {"rmsnorm", {launch_rmsnorm, -1}},
-        {"batch_split_q", {launch_batch_split_q, -1}},
-        {"attention_online_int8_q32_k256_r2", {launch_online_int8, 3}},
-        {"attention_online_int8", {launch_online_int8, 3}},
-        {"attention_online_int8_q32_k128", {launch_online_int8, 3}},
-        {"attention_decode_int8", {launch_decode_int8, 3}},
-        {"attention_decode_append_int8", {launch_decode_append_int8, 3}},
-        {"attention_verify_int8", {launch_verify_int8, 3}},
-        {"attention_online_q32_k256_s8_g8_r2", {launch_online_fp16, 3}},
-        {"batch_rope", {launch_batch_rope_half, -1}},
-        {"attention_prepare_fused", {launch_prepare_fused_half, -1}},
-        {"batch_attention_scores_int8", {launch_scores_int8, 0}},
-        {"attention_softmax", {launch_softmax, 1}},
-        {"batch_attention_values_int8", {launch_values_int8, 2}},
-    };
-    return table;
-}
+// The kernels by name, the ones of every token and chunk first.
+const Entry kRegistry[] = {
+    {"attention_decode_append_int8", launch_decode_append_int8, 3},
+    {"attention_decode_int8", launch_decode_int8, 3},
+    {"attention_verify_int8", launch_verify_int8, 3},
+    {"attention_prepare_fused_int8", launch_prepare_fused_int8, -1},
+    {"attention_online_int8_q32_k256_r2", launch_online_int8, 3},
+    {"batch_rope_int8", launch_batch_rope_int8, -1},
+    {"kv_store_int8", launch_kv_store_int8, -1},
+    {"attention_query_grouped_half", launch_query_grouped_half, -1},
+    {"rmsnorm", launch_rmsnorm, -1},
+    {"batch_split_q", launch_batch_split_q, -1},
+    {"attention_online_int8", launch_online_int8, 3},
+    {"attention_online_int8_q32_k128", launch_online_int8, 3},
+    {"attention_online_q32_k256_s8_g8_r2", launch_online_fp16, 3},
+    {"batch_rope", launch_batch_rope_half, -1},
+    {"attention_prepare_fused", launch_prepare_fused_half, -1},
+    {"batch_attention_scores_int8", launch_scores_int8, 0},
+    {"attention_softmax", launch_softmax, 1},
+    {"batch_attention_values_int8", launch_values_int8, 2},
+};
 
 Buffer *as_buffer(Context *c, void *handle) {
     Buffer *b = static_cast<Buffer *>(handle);
@@ -193,6 +197,17 @@ Buffer *as_buffer(Context *c, void *handle) {
 
 hipStream_t context_stream(Context &c) { return c.stream; }
 int context_cus(Context &c) { return c.cus; }
+
+const RopeFreq &context_rope(Context &c, float theta) {
+    uint32_t bits;
+    memcpy(&bits, &theta, sizeof bits);
+    if (!c.rope_valid || bits != c.rope_theta) {
+        c.rope = rope_frequencies(theta);
+        c.rope_theta = bits;
+        c.rope_valid = true;
+    }
+    return c.rope;
+}
 
 void *context_workspace(Context &c, uint64_t bytes) {
     if (c.noalloc) {
@@ -470,8 +485,11 @@ int dispatch(Context *c, const char *name, void **buffers, const uint64_t *offse
              uint32_t tx, uint32_t ty, uint32_t tz, void *indirect, bool noalloc) {
     if (!c->active) return fail(c, "boot_dispatch requires an active command");
     const Entry *entry = nullptr;
-    for (auto &item : registry())
-        if (name && strcmp(item.first.c_str(), name) == 0) entry = &item.second;
+    for (const Entry &item : kRegistry)
+        if (name && strcmp(item.name, name) == 0) {
+            entry = &item;
+            break;
+        }
     if (!entry) return fail(c, std::string("Unknown kernel: ") + (name ? name : "(null)"));
     if (indirect) return fail(c, std::string(name) + ": indirect dispatch is not supported by INT8 kernels");
     if (count < 0 || count > 31) return fail(c, std::string(name) + ": invalid binding count");
