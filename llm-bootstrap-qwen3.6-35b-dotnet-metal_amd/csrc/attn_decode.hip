@@ -469,13 +469,6 @@ __device__ inline float xl_max32(float x) {
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
     return fmaxf(a, b);
 }
-// x of lane l ^ 8 (the other half of its 16-lane row) by a DPP rotation of the row by 8
-__device__ inline float xl_swap8(float x) {
-    float y;
-    asm volatile("s_nop 1\n\tv_mov_b32_dpp %0, %1 row_ror:8 row_mask:0xf bank_mask:0xf" : "=v"(y) : "v"(x));
-    return y;
-}
-
 // Every element's maximum over the wave: rotations of the 16-lane rows by DPP (the steps of
 // several elements interleave, covering each other's wait states), then across the rows
 template <int N>
@@ -520,6 +513,49 @@ __device__ inline void add_row_partner8(floatx4 &a, floatx4 &b) {
         : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
     a = floatx4{r0, r1, r2, r3};
     b = floatx4{r4, r5, r6, r7};
+}
+
+// The same for four integers (MFMA results scaled by ordinary VALU instructions)
+__device__ inline void add_row_partner8(int (&a)[4]) {
+    int r0, r1, r2, r3;
+    asm volatile(
+        "s_nop 1\n\t"
+        "v_add_u32_dpp %0, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %1, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %2, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %3, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1"
+        : "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3)
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
+    a[0] = r0;
+    a[1] = r1;
+    a[2] = r2;
+    a[3] = r3;
+}
+
+// The three INT8 parts of four query elements of a head whose largest magnitude is amax, four codes a
+// word. z = q / s_q lies in [-127, 127]; q1 = rint(z), q2 = rint(254 r1) of the remainder r1 = z - q1
+// (|r1| <= 1/2) and q3 = rint(254 r2) of r2 = 254 r1 - q2. Adding 1.5 x 2^23 rounds to an integer
+// whose low byte is its two's complement code: 7 operations an element where rint, clamp, convert and
+// pack took 20 (an instruction of 8 waves on 4 SIMDs: 8 cycles).
+__device__ __attribute__((always_inline)) inline void query_parts(const float4 &q, float amax, uint32_t (&w)[3]) {
+    constexpr float kMagic = 12582912.0f;
+    const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
+    const float xs[4] = {q.x, q.y, q.z, q.w};
+    uint32_t t[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float t1 = fmaf(xs[e], inv, kMagic), q1 = t1 - kMagic, r1 = fmaf(xs[e], inv, -q1);
+        const float t2 = fmaf(r1, 254.0f, kMagic), q2 = t2 - kMagic, r2 = fmaf(r1, 254.0f, -q2);
+        const float t3 = fmaf(r2, 254.0f, kMagic);
+        t[0][e] = __builtin_bit_cast(uint32_t, t1);
+        t[1][e] = __builtin_bit_cast(uint32_t, t2);
+        t[2][e] = __builtin_bit_cast(uint32_t, t3);
+    }
+#pragma unroll
+    for (int part = 0; part < 3; part++)
+        w[part] = __builtin_amdgcn_perm(t[part][1], t[part][0], 0x0c0c0400u) |
+                  __builtin_amdgcn_perm(t[part][3], t[part][2], 0x04000c0cu);
 }
 
 // One chunk of one KV group in flight, K and V in separate register sets (K is staged
@@ -667,6 +703,12 @@ __device__ __attribute__((always_inline)) inline void patch_v(VRegs &r, int tid,
 // vs_ref split into FP16 hi + lo; vs_ref, the split's largest V scale, keeps Px below
 // 256 and multiplies the result once. Lane l holds MFMA column n = l % 16 and
 // token/k group qq = l / 16.
+// Up to about 16000 tokens a split is one chunk and the kernel one chunk's latency, most of it issue
+// (an instruction of all eight waves takes 8 cycles of a SIMD): the query's parts are built by a head
+// per wave, the prologue has one barrier (two for the work-group that appends), the first chunk's
+// operands are made once, after its maxima, and masks are applied only in a row's last chunk. At 777
+// tokens 8.9 -> 7.2 us, at 9000 9.4 -> 8.0, at 30000 13.7 -> 12.0; at 131072, where the stream bounds
+// it, 28.9 -> 27.2 us (5.0 TB/s).
 template <bool kHalfQ>
 __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     typedef int v4i __attribute__((ext_vector_type(4)));
@@ -674,18 +716,18 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     // the chunk buffers
     __shared__ __attribute__((aligned(16))) unsigned char arena[2 * sizeof(ChunkLds)];
     ChunkLds *bufs = reinterpret_cast<ChunkLds *>(arena);
-    __shared__ float chunk_top[2][kDecodeWaves][16], wave_l[kDecodeWaves][16];
-    __shared__ uint2 pshare[2][kDecodeWaves][64];   // each wave's P operands, by chunk parity
-    __shared__ float kscale[kMaxSplitTokens], vscale[kMaxSplitTokens];
-    __shared__ float red[kDecodeWaves], qmax[4][8];
-    // append mode: rotated dims 0..63 of the group's 8 query heads, and the new token's codes
-    // (K row, V column) and scales
-    __shared__ __attribute__((aligned(16))) float qrot0[8][64];
+    __shared__ __attribute__((aligned(16))) float chunk_top[2][16][kDecodeWaves];
+    __shared__ float wave_l[kDecodeWaves][16];
+    // each wave's P operands, by chunk parity: [wave][column][four of its tokens], as rows_int8_kernel
+    __shared__ __attribute__((aligned(16))) uint2 pshare[2][kDecodeWaves][16][4];
+    __shared__ __attribute__((aligned(16))) float kscale[kMaxSplitTokens], vscale[kMaxSplitTokens];
+    __shared__ float red[kDecodeWaves], qmax[8];
+    // append mode: the new token's codes (K row, V column) and scales
     __shared__ __attribute__((aligned(16))) uint8_t fresh_k[256], fresh_v[256];
     __shared__ float fresh_scale[2];
-    // INT8 query operands [set][MFMA c][lane] (set 0: q1 | q2 columns, set 1: q3), built once
-    // and read into registers before the chunk loop. They sit in the V half of chunk buffer
-    // 1, which is first written in phase 1, after the barrier that ends phase 0: by then every
+    // INT8 query operands [set][MFMA c][slot] (set 0: q1 | q2 columns, set 1: q3 in columns n < 8),
+    // lane (n, qq)'s in slot 16 qq + (n ^ (4 c + qq)) as in rows_int8_kernel, built once and read
+    // into registers before the chunk loop. They sit in the V half of chunk buffer 1, which is first written in phase 1, after the barrier that ends phase 0: by then every
     // wave has read its operands.
     v4i(*qlds)[4][64] = reinterpret_cast<v4i(*)[4][64]>(&bufs[1].v[0][0]);
     static_assert(2 * 4 * 64 * sizeof(v4i) <= sizeof(ChunkLds::v), "query operands exceed the V half of a buffer");
@@ -710,41 +752,31 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     // indices past the split repeat its last token, a cache hit)
     uint32_t last = (end > begin ? end : length) - 1;
     if (p.append && last == p.pos && p.pos > 0) last = p.pos - 1;   // its stored scales are stale
-    float ksv[kMaxSplitTokens / 512], vsv[kMaxSplitTokens / 512];
+    constexpr int kPasses = kMaxSplitTokens / 512;   // (a pass past the split is skipped: uniform)
+    float ksv[kPasses], vsv[kPasses];
 #pragma unroll
-    for (int it = 0; it < kMaxSplitTokens / 512; it++) {
+    for (int it = 0; it < kPasses; it++) {
+        if (it > 0 && begin + 512 * it >= end) break;
         const size_t at = (size_t)min(begin + tid + 512 * it, last) * 2 + g;
         ksv[it] = p.ks[at];
         vsv[it] = p.vs[at];
     }
-    // query chunk c = wave % 4: lane (n, qq) takes dims 64c + 16qq + [0, 16) of head
-    // n % 8 (waves 4-7 load the same chunks and only waves 0-3 publish them)
-    const int chunk = wave & 3;
-    float4 x[4];
-    if constexpr (kHalfQ) {
-        // the prefill path's grouped FP16 query, [(g rows + row) 8 + head][256]: exact in FP32
-        const _Float16 *qs = p.qh + (((size_t)g * p.rows + row) * 8 + head) * 256 + 64 * chunk + 16 * qq;
-        const half8 a = *reinterpret_cast<const half8 *>(qs), b = *reinterpret_cast<const half8 *>(qs + 8);
-        x[0] = make_float4((float)a[0], (float)a[1], (float)a[2], (float)a[3]);
-        x[1] = make_float4((float)a[4], (float)a[5], (float)a[6], (float)a[7]);
-        x[2] = make_float4((float)b[0], (float)b[1], (float)b[2], (float)b[3]);
-        x[3] = make_float4((float)b[4], (float)b[5], (float)b[6], (float)b[7]);
+    // head `wave` of the group in rope4's layout (dims 4 lane .. +3), and in append mode the new
+    // token's K and V of the group (from the query itself when there is no new token: a fixed count
+    // of loads keeps the counter waits exact)
+    float4 rq;
+    if constexpr (kHalfQ) {   // the prefill path's grouped FP16 query, exact in FP32
+        const half4 a = *reinterpret_cast<const half4 *>(p.qh + (((size_t)g * p.rows + row) * 8 + wave) * 256 + 4 * lane);
+        rq = make_float4((float)a[0], (float)a[1], (float)a[2], (float)a[3]);
     } else {
-        const float *qs = p.q + ((size_t)row * 16 + g * 8 + head) * 256 + 64 * chunk + 16 * qq;
-#pragma unroll
-        for (int f = 0; f < 4; f++) x[f] = *reinterpret_cast<const float4 *>(qs + 4 * f);
+        rq = *reinterpret_cast<const float4 *>(p.q + ((size_t)row * 16 + g * 8 + wave) * 256 + 4 * lane);
     }
-    // append mode: head `wave` of the group in rope4's layout (dims 4 lane .. +3) and the new
-    // token's K and V of the group. Loaded in every mode and every wave (from the query itself
-    // when there is no new token): a fixed count of loads keeps the counter waits exact.
-    // (the FP16 query path has no FP32 query and no new token: its first 2 KB, in range for any
-    // row count, stand in for these unused loads)
-    const float *qf = kHalfQ ? reinterpret_cast<const float *>(p.qh) : p.q;
-    const float *knew = p.append ? p.knew : qf, *vnew = p.append ? p.vnew : qf;
-    const float4 rq = *reinterpret_cast<const float4 *>(
-        kHalfQ ? qf + 4 * lane : p.q + ((size_t)row * 16 + g * 8 + wave) * 256 + 4 * lane);
-    const float4 nk = *reinterpret_cast<const float4 *>(knew + (size_t)g * 256 + 4 * lane);
-    const float4 nv = *reinterpret_cast<const float4 *>(vnew + (size_t)g * 256 + 4 * lane);
+    float4 nk = rq, nv = rq;
+    if constexpr (!kHalfQ) {
+        const float *knew = p.append ? p.knew : p.q, *vnew = p.append ? p.vnew : p.q;
+        nk = *reinterpret_cast<const float4 *>(knew + (size_t)g * 256 + 4 * lane);
+        nv = *reinterpret_cast<const float4 *>(vnew + (size_t)g * 256 + 4 * lane);
+    }
     // every wave's small loads enter the CU's memory pipeline before any chunk load
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
@@ -756,16 +788,15 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     load_k(kb, p, g, begin, 1, nchunks, length, tid);
     load_v(vb, p, g, begin, 1, nchunks, tid);
 
-    float vmax = 0.0f;
+    float vmax[1] = {0.0f};
     if (p.append) {
         // the same rotation (and, for the new token, quantization) as batch_rope_int8
         // (kv_store.hip), so the cache bytes and the rotated query match it bit for bit
         const float ifreq = lane_inv_freq(p.freq);
         const Rope4 r = rope_angles(p.pos, lane, ifreq);
-        const float4 z = rope4(rq, lane, r);
-        if (lane < 16) *reinterpret_cast<float4 *>(&qrot0[wave][4 * lane]) = z;
+        rq = rope4(rq, lane, r);
         if (owner) {
-            *reinterpret_cast<float4 *>(p.rotated + ((size_t)g * 8 + wave) * 256 + 4 * lane) = z;
+            *reinterpret_cast<float4 *>(p.rotated + ((size_t)g * 8 + wave) * 256 + 4 * lane) = rq;
             const uint64_t vector = (uint64_t)p.pos * 2 + g;
             if (wave == 0) {
                 const float4 kz = rope4(nk, lane, r);
@@ -794,125 +825,91 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
                     p.vs_out[vector] = va / 127.0f;
                     fresh_scale[1] = va / 127.0f;
                 }
-                vmax = va / 127.0f;   // the new token joins the split's largest V scale
             }
+            __syncthreads();   // the fresh codes and scales are in LDS (owner is work-group-uniform)
         }
     }
-
-    // ---- K scales of the split (this group) into LDS, vs_ref = the maximum of its V scales;
-    // the per-head maxima of the query chunks
-#pragma unroll
-    for (int it = 0; it < kMaxSplitTokens / 512; it++) {
-        const uint32_t e = tid + 512 * it;   // < kMaxSplitTokens; entries past the split are never read
-        // entries past the split are zero (selected after the unconditional loads); in append
-        // mode the new token's entry is set from its fresh scale below
-        const bool inside = begin + e < end && (int)e != e_new;
-        kscale[e] = inside ? ksv[it] * (kLog2e / 16.0f) : 0.0f;
-        vmax = fmaxf(vmax, inside ? vsv[it] : 0.0f);
-    }
-    if (p.append) {
-        __syncthreads();   // the rotated query dims and the fresh codes and scales are in LDS
-        if (chunk == 0) {
-            // dims 16 qq + [0, 16) of head n % 8: the rotated values
-#pragma unroll
-            for (int f = 0; f < 4; f++) x[f] = *reinterpret_cast<const float4 *>(&qrot0[head][16 * qq + 4 * f]);
-        }
-        if (tid == 0 && owner) kscale[e_new] = fresh_scale[0] * (kLog2e / 16.0f);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
-    if (lane == 0) red[wave] = vmax;
-    float amax = 0.0f;
-#pragma unroll
-    for (int f = 0; f < 4; f++) amax = fmaxf(amax, fmaxf(fmaxf(fabsf(x[f].x), fabsf(x[f].y)), fmaxf(fabsf(x[f].z), fabsf(x[f].w))));
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-    if (lane < 8 && wave < 4) qmax[wave][lane] = amax;
-    __syncthreads();
-    float vs_ref = red[0];
-#pragma unroll
-    for (int w = 1; w < kDecodeWaves; w++) vs_ref = fmaxf(vs_ref, red[w]);
-    const float vs_inv = vs_ref > 0.0f ? 1.0f / vs_ref : 0.0f;
-    // the split's V scales times 1 / vs_ref, the factor of the probability operand (entries past
-    // the split zero, the new token's from its fresh scale); the barrier before phase 0 publishes them
-#pragma unroll
-    for (int it = 0; it < kMaxSplitTokens / 512; it++) {
-        const uint32_t e = tid + 512 * it;
-        const float s = (int)e == e_new ? fresh_scale[1] : vsv[it];
-        vscale[e] = begin + e < end ? s * vs_inv : 0.0f;
-    }
-    // ---- INT8 query operands of chunk c = wave: q ~= s_q (q1 + q2 / 254 + q3 / 254^2).
-    // z = q / s_q lies in [-127, 127]; q1 = rint(z) and r1 = z - q1 (exact, |r1| <= 1/2);
-    // q2 = rint(254 r1) and r2 = 254 r1 - q2 (one rounding, |r2| <= 1/2 + 2^-17);
-    // q3 = rint(254 r2). Set 0 holds q1 in columns n < 8 and q2 in n >= 8, set 1 q3 in both.
-    const float qabs = fmaxf(fmaxf(qmax[0][head], qmax[1][head]), fmaxf(qmax[2][head], qmax[3][head]));
-    const float qsc = qabs * (1.0f / 127.0f);   // s_q of the lane's head
+    // ---- the INT8 parts of head `wave`, one lane's four dimensions (as rows_int8_kernel: each wave
+    // one head, where every wave built a quarter of all eight and the maxima met behind a barrier)
     {
-        const float inv = qabs > 0.0f ? 127.0f / qabs : 0.0f;
-        auto code = [](float q) { return (uint32_t)(uint8_t)(int8_t)(int)fminf(fmaxf(q, -127.0f), 127.0f); };
-        uint32_t w[4], w3[4];
-#pragma unroll
-        for (int f = 0; f < 4; f++) {
-            const float xs[4] = {x[f].x, x[f].y, x[f].z, x[f].w};
-            w[f] = w3[f] = 0;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float z = xs[e] * inv, q1 = rintf(z), r1 = z - q1;
-                const float q2 = rintf(r1 * 254.0f);
-                const float r2 = fmaf(r1, 254.0f, -q2);
-                const float q3 = rintf(r2 * 254.0f);
-                w[f] |= code(lo_col ? q2 : q1) << (8 * e);
-                w3[f] |= code(q3) << (8 * e);
-            }
-        }
-        if (wave < 4) {
-            qlds[0][wave][lane] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-            qlds[1][wave][lane] = v4i{(int)w3[0], (int)w3[1], (int)w3[2], (int)w3[3]};
-        }
+        float amax[1] = {fmaxf(fmaxf(fabsf(rq.x), fabsf(rq.y)), fmaxf(fabsf(rq.z), fabsf(rq.w)))};
+        wave_allmax(amax);
+        uint32_t w[3];
+        query_parts(rq, amax[0], w);
+        const int c = lane >> 4, bq = (lane >> 2) & 3, mix = 4 * c + bq;
+        reinterpret_cast<uint32_t *>(&qlds[0][c][16 * bq + (wave ^ mix)])[lane & 3] = w[0];
+        reinterpret_cast<uint32_t *>(&qlds[0][c][16 * bq + ((8 + wave) ^ mix)])[lane & 3] = w[1];
+        reinterpret_cast<uint32_t *>(&qlds[1][c][16 * bq + (wave ^ mix)])[lane & 3] = w[2];
+        if (lane == 0) qmax[wave] = amax[0];
     }
+    // ---- the split's scales (this group) into LDS, vs_ref = the maximum of its V scales; entries past
+    // the split are zero, the new token's from its fresh scales
+#pragma unroll
+    for (int it = 0; it < kPasses; it++) {
+        if (it > 0 && begin + 512 * it >= end) break;
+        const uint32_t e = tid + 512 * it;
+        const bool inside = begin + e < end, fresh = (int)e == e_new;
+        const float sk = fresh ? fresh_scale[0] : ksv[it], sv = fresh ? fresh_scale[1] : vsv[it];
+        kscale[e] = inside ? sk * (kLog2e / 16.0f / 254.0f) : 0.0f;   // a dot's unit is 1 / 254 (below)
+        vscale[e] = inside ? sv : 0.0f;
+        vmax[0] = fmaxf(vmax[0], inside ? sv : 0.0f);
+    }
+    wave_allmax(vmax);
+    if (lane == 0) red[wave] = vmax[0];
     // K of chunk 0 into buffer 0 and K of chunk 2 into the registers it leaves
     if (jn == 0) patch_k(ka, tid, tn, reinterpret_cast<const uint4 *>(fresh_k));
     store_k(bufs[0], ka, tid);
     load_k(ka, p, g, begin, 2, nchunks, length, tid);
     __syncthreads();
+    float vs_ref = red[0];
+#pragma unroll
+    for (int w = 1; w < kDecodeWaves; w++) vs_ref = fmaxf(vs_ref, red[w]);
+    // operands up to 2^8 times 2^7 stay below FP16's 65504; the factor keeps their lo parts out of its
+    // subnormals
+    const float vs_inv = vs_ref > 0.0f ? 128.0f / vs_ref : 0.0f;
+    vs_ref *= 1.0f / 128.0f;
+    const float qsc = qmax[head] * (1.0f / 127.0f);   // s_q of the lane's head
     v4i qi[4], q3i[4];
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        qi[c] = qlds[0][c][lane];
-        q3i[c] = qlds[1][c][lane];
+        qi[c] = qlds[0][c][16 * qq + (n ^ (4 * c + qq))];
+        q3i[c] = qlds[1][c][16 * qq + (head ^ (4 * c + qq))];
     }
 
     floatx4 o[2];   // O^T tiles dt = 2 wave + i, over every token of the split
     o[0] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     o[1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m = -INFINITY, l = 0.0f;
+    float m = -INFINITY, l = 0.0f, total_prev = 0.0f;   // l: this lane's tokens, summed at the end
+    float dot_prev[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // the previous chunk's dots, for a rebuild of its operands
 
-    // Probabilities of the lane's four tokens against reference ref, as the FP16 hi (column
-    // n < 8) or lo (n >= 8) part of p * vs / vs_ref, published as this wave's P operand in
-    // slot `slot`; total = the column's sum over the wave's 16 tokens.
-    auto probs = [&](const float (&sc)[4], int local0, float ref, float &total, int slot) __attribute__((always_inline)) {
-        // ref = -inf (before the first rescale) gives +inf for unmasked tokens: their chunk
-        // always rescales, which rebuilds the operands and the total before either is read
-        const float refc = fmaxf(ref, -3.0e38f);
-        _Float16 hv[4];
-        total = 0.0f;
+    // Probabilities of the lane's four tokens of chunk j against the running reference, as the FP16 hi
+    // (column n < 8) or lo (n >= 8) part of p * vs / vs_ref, published as this wave's P operand;
+    // total_prev = the lane's sum.
+    auto probs = [&](uint32_t j) __attribute__((always_inline)) {
+        const int local0 = (int)(j * kChunk) + 16 * wave + 4 * qq;   // token offset inside the split
+        const float4 vs4 = *reinterpret_cast<const float4 *>(&vscale[local0]);
+        const float4 ks4 = *reinterpret_cast<const float4 *>(&kscale[local0]);
+        const float vsr[4] = {vs4.x, vs4.y, vs4.z, vs4.w}, ksr[4] = {ks4.x, ks4.y, ks4.z, ks4.w};
+        const float refc = fmaxf(m, -3.0e38f);   // m = -inf only in a column without a score yet
+        float arg[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) arg[r] = fmaf(dot_prev[r], qsc * ksr[r], -refc);
+        if (begin + (j + 1) * kChunk > end)   // uniform: only a row's last chunk holds tokens past its end
+#pragma unroll
+            for (int r = 0; r < 4; r++) arg[r] = begin + local0 + r < end ? arg[r] : -INFINITY;
+        half4 pop;
+        total_prev = 0.0f;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const float prob = __builtin_amdgcn_exp2f(sc[r] - refc);   // 0 for masked tokens
-            total += prob;
-            const float scaled = prob * vscale[local0 + r];
+            const float prob = __builtin_amdgcn_exp2f(arg[r]);   // 0 for masked tokens
+            total_prev += prob;
+            float scaled = prob * (vsr[r] * vs_inv);
+            asm("" : "+v"(scaled));   // one rounded value for both parts (see rows_int8_kernel)
             const _Float16 hi = (_Float16)scaled;
-            hv[r] = lo_col ? (_Float16)(scaled - (float)hi) : hi;
+            pop[r] = lo_col ? (_Float16)(scaled - (float)hi) : hi;
         }
-        total = xl_sum16(total);
-        total = xl_sum32(total);
-        const half4 pop = {hv[0], hv[1], hv[2], hv[3]};
-        pshare[slot][wave][lane] = __builtin_bit_cast(uint2, pop);
+        pshare[j & 1][wave][n][qq] = __builtin_bit_cast(uint2, pop);
     };
-    // the previous chunk's scores, kept for a rebuild of its operands
-    float sc_prev[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    float total_prev = 0.0f;
-    int local_prev = 0;
     // Phase j (one barrier each): finish chunk j - 1 (the rescale decision, then PV), score
     // chunk j, store V of chunk j and K of chunk j + 1, load V of chunk j + 2 and K of chunk
     // j + 3 into the registers just stored. K is staged one chunk ahead of V, so the two
@@ -924,25 +921,26 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     auto finish = [&](uint32_t j) __attribute__((always_inline)) {   // chunk j - 1, j > 0
         {
             const int slot = (j - 1) & 1;
-            float ctop = chunk_top[slot][0][n];
-#pragma unroll
-            for (int w = 1; w < kDecodeWaves; w++) ctop = fmaxf(ctop, chunk_top[slot][w][n]);
-            // every wave reads the same maxima: the branch is uniform over the work-group
-            if (__builtin_amdgcn_ballot_w64(ctop > m + 8.0f) != 0) {
+            const float4 ta = *reinterpret_cast<const float4 *>(&chunk_top[slot][n][0]);
+            const float4 tb = *reinterpret_cast<const float4 *>(&chunk_top[slot][n][4]);
+            const float ctop = fmaxf(fmaxf(fmaxf(ta.x, ta.y), fmaxf(ta.z, ta.w)), fmaxf(fmaxf(tb.x, tb.y), fmaxf(tb.z, tb.w)));
+            // every wave reads the same maxima: the branch is uniform over the work-group. Chunk 0 has
+            // no reference before its maxima: its operands are made here
+            if (j == 1 || __builtin_amdgcn_ballot_w64(ctop > m + 8.0f) != 0) {
                 const float next = fmaxf(m, ctop);
                 const float decay = next == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - next);
                 l *= decay;
                 o[0] *= decay;
                 o[1] *= decay;
                 m = next;
-                probs(sc_prev, local_prev, m, total_prev, slot);   // no wave reads the slot before this branch
+                probs(j - 1);   // no wave reads the slot before this branch
                 __syncthreads();
             }
-            l += total_prev;   // this wave's tokens
+            l += total_prev;
             // O^T[d][n] += V^T[d][t] P[t][n] for this wave's 32 dimensions over the chunk's 128
             // tokens on v_mfma_f32_16x16x32_f16: k-step s takes waves 2s and 2s + 1's tokens (32),
             // lane (n, qq) tokens 8 (qq % 2) .. + 7 of wave 2s + qq / 2, i.e. the published P
-            // operands of lanes n + 32 (qq % 2) and n + 32 (qq % 2) + 16 of that wave and 8 codes
+            // operands 2 (qq % 2) and 2 (qq % 2) + 1 of column n and 8 codes
             // (one 8-byte read) of its V piece. Against 16 MFMAs of 16 tokens with a 4-byte read
             // each: half the MFMAs, dependent steps and V reads (29.6-30.0 against 30.2-30.3 us
             // per layer step at 131073)
@@ -950,8 +948,7 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
 #pragma unroll
             for (int s = 0; s < kDecodeWaves / 2; s++) {
                 const int src = 2 * s + (qq >> 1);
-                const uint2 pa = pshare[slot][src][n + 32 * (qq & 1)], pb = pshare[slot][src][n + 32 * (qq & 1) + 16];
-                const half8 ps = __builtin_bit_cast(half8, make_uint4(pa.x, pa.y, pb.x, pb.y));
+                const half8 ps = *reinterpret_cast<const half8 *>(&pshare[slot][src][n][2 * (qq & 1)]);
 #pragma unroll
                 for (int jj = 0; jj < 2; jj++) {
                     const int d = 16 * (2 * wave + jj) + n;
@@ -981,25 +978,29 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
                 acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, qi[jj], acc, 0, 0, 0);
                 acc3 = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, q3i[jj], acc3, 0, 0, 0);
             }
-            // the partner column n ^ 8 holds the other part of the same head; every dot is
-            // an integer below 2^22 in magnitude, exact in FP32
+            // column n holds the q1 dots (n < 8) or the q2 dots of head n % 8, and the partner column
+            // the other: 254 dot1 + dot2 is an exact integer (|dots| < 2^22), summed over the pair by
+            // one DPP add. The exponent's argument is one fma of the dot (probs), so the score itself,
+            // rounded, is only compared
             const int local0 = (int)(j * kChunk) + 16 * wave + 4 * qq;   // token offset inside the split
-            const uint32_t t0 = begin + (uint32_t)local0;
-            float top = -INFINITY;
+            const float4 ks4 = *reinterpret_cast<const float4 *>(&kscale[local0]);
+            const float ksr[4] = {ks4.x, ks4.y, ks4.z, ks4.w};
+            float score[4];
+            int d12[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) d12[r] = __mul24(acc[r], lo_col ? 1 : 254);
+            add_row_partner8(d12);
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float mine = (float)acc[r], other = xl_swap8(mine);   // exact: |dot| < 2^22
-                const float hi = lo_col ? other : mine, lo = lo_col ? mine : other;
-                const float full = fmaf((float)acc3[r], 1.0f / 64516.0f, fmaf(lo, 1.0f / 254.0f, hi)) * qsc;
-                const float value = t0 + r < end ? full * kscale[local0 + r] : -INFINITY;
-                sc_prev[r] = value;
-                top = fmaxf(top, value);
+                dot_prev[r] = fmaf((float)acc3[r], 1.0f / 254.0f, (float)d12[r]);
+                score[r] = dot_prev[r] * (qsc * ksr[r]);
             }
-            top = xl_max16(top);
-            top = xl_max32(top);
-            local_prev = local0;
-            probs(sc_prev, local0, m, total_prev, j & 1);
-            if (qq == 0) chunk_top[j & 1][wave][n] = top;
+            if (begin + (j + 1) * kChunk > end)
+#pragma unroll
+                for (int r = 0; r < 4; r++) score[r] = begin + local0 + r < end ? score[r] : -INFINITY;
+            const float top = xl_max32(xl_max16(fmaxf(fmaxf(score[0], score[1]), fmaxf(score[2], score[3]))));
+            if (qq == 0) chunk_top[j & 1][n][wave] = top;
+            if (j > 0) probs(j);
         }
         if ((int)j == jn) patch_v(rv, tid, tn, fresh_v);
         store_v(bufs[j & 1], rv, tid);
@@ -1041,28 +1042,28 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     // column n + 8 of each head joins its hi column n in registers (the DPP adds take MFMA
     // results as inline-assembly operands, for which the compiler inserts no wait states:
     // cover them here), then lanes n < 8 hold tile 2 wave and lanes n >= 8 tile 2 wave + 1.
+    l = xl_sum32(xl_sum16(l));
     if (qq == 0) wave_l[wave][n] = l;
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
     __builtin_amdgcn_sched_barrier(0);
     add_row_partner8(o[0], o[1]);
-    __syncthreads();
-    float lw = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kDecodeWaves; w++) lw += wave_l[w][head];
     const bool upper = n >= 8;
     const int d0 = 16 * (2 * wave + (upper ? 1 : 0)) + 4 * qq;
     const int h = head;
-    const float mw = m;
     floatx4 res = upper ? o[1] : o[0];
     float4 acc = make_float4(res[0] * vs_ref, res[1] * vs_ref, res[2] * vs_ref, res[3] * vs_ref);
     if (p.splits == 1) {
         // gate and y need only 4-byte alignment
         // (the four gate loads go out before the first store: the compiler cannot tell y from gate)
         const size_t at = ((size_t)row * 16 + g * 8 + h) * 256 + d0;
-        const float inv = 1.0f / lw;
         const float g0 = p.gate[at + 0], g1 = p.gate[at + 1], g2 = p.gate[at + 2], g3 = p.gate[at + 3];
         asm volatile("" ::"v"(g0), "v"(g1), "v"(g2), "v"(g3) : "memory");
+        __syncthreads();
+        float lw = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kDecodeWaves; w++) lw += wave_l[w][head];
+        const float inv = 1.0f / lw;
         p.y[at + 0] = acc.x * inv * sigmoidf(g0);
         p.y[at + 1] = acc.y * inv * sigmoidf(g1);
         p.y[at + 2] = acc.z * inv * sigmoidf(g2);
@@ -1070,9 +1071,13 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
         return;
     }
     float *part = p.partial + (((size_t)row * 2 + g) * p.splits + split) * kPartialFloats;
-    *reinterpret_cast<float4 *>(part + h * 256 + d0) = acc;
+    *reinterpret_cast<float4 *>(part + h * 256 + d0) = acc;   // needs no other wave's l
+    __syncthreads();
     if (wave == 0 && lane < 8) {
-        part[2048 + h] = mw;
+        float lw = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kDecodeWaves; w++) lw += wave_l[w][head];
+        part[2048 + h] = m;
         part[2056 + h] = lw;
     }
 }
@@ -1310,39 +1315,21 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     load_k(kb, 1);
     load_v(vb, 1);
 
-    // ---- the query's INT8 parts. z = q / s_q lies in [-127, 127]; q1 = rint(z), q2 = rint(254 r1) of
-    // the remainder r1 = z - q1 (|r1| <= 1/2) and q3 = rint(254 r2) of r2 = 254 r1 - q2. Adding 1.5 x
-    // 2^23 rounds to an integer whose low byte is its two's complement code: 7 operations an element
-    // where rint, clamp, convert and pack took 20 (8 waves on 4 SIMDs: 8 cycles each).
+    // ---- the query's INT8 parts
     float amax[kRowsPer];
 #pragma unroll
     for (int r = 0; r < kRowsPer; r++) amax[r] = fmaxf(fmaxf(fabsf(x[r].x), fabsf(x[r].y)), fmaxf(fabsf(x[r].z), fabsf(x[r].w)));
     wave_allmax(amax);
 #pragma unroll
     for (int r = 0; r < kRowsPer; r++) {
-        constexpr float kMagic = 12582912.0f;
-        const float inv = amax[r] > 0.0f ? 127.0f / amax[r] : 0.0f;
-        const float xs[4] = {x[r].x, x[r].y, x[r].z, x[r].w};
-        uint32_t t[3][4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float t1 = fmaf(xs[e], inv, kMagic), q1 = t1 - kMagic, r1 = fmaf(xs[e], inv, -q1);
-            const float t2 = fmaf(r1, 254.0f, kMagic), q2 = t2 - kMagic, r2 = fmaf(r1, 254.0f, -q2);
-            const float t3 = fmaf(r2, 254.0f, kMagic);
-            t[0][e] = __builtin_bit_cast(uint32_t, t1);
-            t[1][e] = __builtin_bit_cast(uint32_t, t2);
-            t[2][e] = __builtin_bit_cast(uint32_t, t3);
-        }
-        // dimension 4 lane: step c, block qq (of the operand's lanes), word lane % 4 of its 16 bytes
+        uint32_t w[3];
+        query_parts(x[r], amax[r], w);
+        // dimension 4 lane: step c, block bq (of the operand's lanes), word lane % 4 of its 16 bytes
         const int c = lane >> 4, bq = (lane >> 2) & 3, col = 8 * (r & 1) + wave;
         const int slot = 16 * bq + (col ^ (4 * c + bq));
-#pragma unroll
-        for (int part = 0; part < 3; part++) {
-            const uint32_t lo = __builtin_amdgcn_perm(t[part][1], t[part][0], 0x0c0c0400u);
-            const uint32_t hi = __builtin_amdgcn_perm(t[part][3], t[part][2], 0x04000c0cu);
-            uint32_t *dst = reinterpret_cast<uint32_t *>(part < 2 ? &qlds[r >> 1][part][c][slot] : &q3lds[r >> 1][c][slot]);
-            dst[lane & 3] = lo | hi;
-        }
+        reinterpret_cast<uint32_t *>(&qlds[r >> 1][0][c][slot])[lane & 3] = w[0];
+        reinterpret_cast<uint32_t *>(&qlds[r >> 1][1][c][slot])[lane & 3] = w[1];
+        reinterpret_cast<uint32_t *>(&q3lds[r >> 1][c][slot])[lane & 3] = w[2];
         if (lane == 0) qmax[r >> 1][col] = amax[r];
     }
     // ---- scales of the split into LDS, the work-group's largest V scale
