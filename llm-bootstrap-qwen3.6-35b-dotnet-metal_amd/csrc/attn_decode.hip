@@ -1156,10 +1156,10 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float *__rest
 // prefill chunks over short key ranges (grouped FP16 query). The
 // decode kernel above gives each row a work-group of its own, so R rows read, stage and convert
 // the cache R times, and the three-kernel reader (five launches) writes every score to memory and
-// reads it back twice. Per layer, with the combine, against the reader: 8 rows after 1500 keys 14.9
-// (40.0) us, where either is launches and one chunk's latency; 4 rows after 30000 keys 24.4 (47.6)
-// us, 1.3 TB/s of cache: bound by the vector work of a chunk (conversions, exponentials, P) and the
-// start of a work-group, not by the stream.
+// reads it back twice. Per layer, with the combine, against the reader: 8 rows after 1500 keys 12.8
+// (40.0) us, where either is launches and one chunk's latency; 4 rows after 30000 keys 21.9 (47.6)
+// us, 1.4 TB/s of cache: bound by the issue of a chunk's vector and matrix work and the start of a
+// work-group, not by the stream.
 //
 // Grid: (split, KV group) pairs x row blocks, one 8-wave work-group per CU; the row blocks of a pair
 // are 8 blocks apart, on one XCD, whose L2 serves the second and later ones. A split is split_chunks
@@ -1236,7 +1236,7 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     }
     const uint32_t nchunks = (end - begin + kChunk - 1) / kChunk;
 
-    // ---- the small loads first, then the first two chunks (as decode_int8_kernel)
+    // ---- the small loads first, then the first chunk (as decode_int8_kernel)
     const uint32_t last = end - 1;
     // (the scales of a split of up to 512 tokens in one load each: the counts of further passes are
     // uniform branches)
@@ -1272,27 +1272,21 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         if constexpr (kOnce) return load_piece(at);
         return *reinterpret_cast<const uint4 *>(at);
     };
-    // K rows 16 wave + 4 i + lane / 16 of chunk idx, piece lane % 16; V segments as load_v. Past the
-    // last chunk (only the prologue's second load) every lane reads one line of the first.
+    // K rows 16 wave + 4 i + lane / 16 of chunk idx, piece lane % 16; V segments as decode_int8_kernel's
     auto load_k = [&](KRegs &r, uint32_t idx) __attribute__((always_inline)) {
-        const bool real = idx < nchunks;
-        const uint32_t t = begin + (real ? idx * kChunk + 16 * wave + (lane >> 4) : 0u), step = real ? 4 : 0;
-        const int8_t *base = p.k + (size_t)g * 256 + 16 * (real ? lane & 15 : 0);
+        const uint32_t t = begin + idx * kChunk + 16 * wave + (lane >> 4);
+        const int8_t *base = p.k + (size_t)g * 256 + 16 * (lane & 15);
         r.k0 = load16(base + (size_t)min(t, last) * 512);
-        r.k1 = load16(base + (size_t)min(t + step, last) * 512);
-        r.k2 = load16(base + (size_t)min(t + 2 * step, last) * 512);
-        r.k3 = load16(base + (size_t)min(t + 3 * step, last) * 512);
+        r.k1 = load16(base + (size_t)min(t + 4, last) * 512);
+        r.k2 = load16(base + (size_t)min(t + 8, last) * 512);
+        r.k3 = load16(base + (size_t)min(t + 12, last) * 512);
     };
     auto load_v = [&](VRegs &r, uint32_t idx) __attribute__((always_inline)) {
-        const bool real = idx < nchunks;
-        const uint32_t c0 = begin + (real ? idx * kChunk : 0u);
-        const int lt = real ? tid : 0;
-        const int8_t *vrow = p.v + value_index((uint64_t)c0 * 2 + g, 0) + (size_t)(lt >> 3) * 256 + 16 * (lt & 7);
-        const size_t step = real ? 64 * 256 : 0;
+        const int8_t *vrow = p.v + value_index((uint64_t)(begin + idx * kChunk) * 2 + g, 0) + (size_t)(tid >> 3) * 256 + 16 * (tid & 7);
         r.v0 = load16(vrow);
-        r.v1 = load16(vrow + step);
-        r.v2 = load16(vrow + 2 * step);
-        r.v3 = load16(vrow + 3 * step);
+        r.v1 = load16(vrow + 64 * 256);
+        r.v2 = load16(vrow + 128 * 256);
+        r.v3 = load16(vrow + 192 * 256);
     };
     auto store_k = [&](const KRegs &r) __attribute__((always_inline)) {
         const int t = lane >> 4, c = lane & 15;
@@ -1308,12 +1302,13 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         vbuf[slot][d + 128][vp] = r.v2;
         vbuf[slot][d + 192][vp] = r.v3;
     };
-    KRegs ka, kb;   // K of even / odd chunks
-    VRegs va, vb;   // V of even / odd chunks
-    load_k(ka, 0);
-    load_v(va, 0);
-    load_k(kb, 1);
-    load_v(vb, 1);
+    // One register set each for K and V: a chunk's loads have a whole phase (about 2 us) to arrive. A
+    // second set, 32 registers that the operand reads then run ahead in, measured slower: 4 rows after
+    // 1500 keys 9.5 against 8.5 us, after 30000 19.1 against 17.6, 1 row after 100000 22.7 against 20.9.
+    KRegs rk;
+    VRegs rv;
+    load_k(rk, 0);
+    load_v(rv, 0);
 
     // ---- the query's INT8 parts
     float amax[kRowsPer];
@@ -1344,8 +1339,8 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     }
     wave_allmax(vmax);
     if (lane == 0) red[wave] = vmax[0];
-    store_k(ka);
-    if (2 < nchunks) load_k(ka, 2);
+    store_k(rk);
+    if (1 < nchunks) load_k(rk, 1);
     __syncthreads();
     // row i of the block sees the tokens before first_end and vnew[0 .. i - 1], where the split holds them
     float vcum = red[0];
@@ -1382,7 +1377,14 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
 #pragma unroll
             for (int c = 0; c < 4; c++) qi[ct][part][c] = qlds[ct][part][c][16 * qq + (n ^ (4 * c + qq))];
 
-    floatx4 o[2][CT];   // O^T: dimensions 32 wave + 16 dt + 4 qq + r of column n
+    // O^T of the wave's 32 dimensions. A prefill chunk holds it as one 32x32 tile, element e of a lane
+    // being dimension 32 wave + 8 (e / 4) + 4 (lane / 32) + e % 4 of column lane % 32 (tile oct, column
+    // n); verify rows, which must come out the same in one tile and in two, as 16x16 tiles
+    constexpr bool kWide = kHalfQ;
+    static_assert(!kWide || CT == 2, "a 32x32 tile holds two tiles' columns");
+    const int oct = (lane >> 4) & 1;
+    floatx16 ow;
+    floatx4 o[2][CT];   // 16x16: dimensions 32 wave + 16 dt + 4 qq + r of column n
     float m[CT], l[CT], total_prev[CT], dot_prev[CT][4];   // l: this lane's tokens, summed over lanes at the end
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) {
@@ -1431,8 +1433,10 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
             pshare[slot][ct][1][wave][n][qq] = __builtin_bit_cast(uint2, lo);
         }
     };
+#pragma unroll
+    for (int e = 0; e < 16; e++) ow[e] = 0.0f;
     // the phases of decode_int8_kernel: finish chunk j - 1, score chunk j, stage V of chunk j and K of
-    // chunk j + 1, load V of chunk j + 2 and K of chunk j + 3; one barrier each
+    // chunk j + 1, load V of chunk j + 1 and K of chunk j + 2; one barrier each
     auto finish = [&](uint32_t j) __attribute__((always_inline)) {
         const int slot = (j - 1) & 1;
         float ctop[CT];
@@ -1448,64 +1452,115 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         // columns that passed the bound change (the others' factor is 1 and their operands the same).
         // Chunk 0 has no reference before its maxima: its operands are made here
         if (j == 1 || __builtin_amdgcn_ballot_w64(raise) != 0) {
+            float decay[CT];
 #pragma unroll
             for (int ct = 0; ct < CT; ct++) {
                 const float next = ctop[ct] > m[ct] + 8.0f ? ctop[ct] : m[ct];
-                const float decay = next == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[ct] - next);
-                l[ct] *= decay;
-                o[0][ct] *= decay;
-                o[1][ct] *= decay;
+                decay[ct] = next == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[ct] - next);
+                l[ct] *= decay[ct];
                 m[ct] = next;
+            }
+            if constexpr (kWide) {
+                const float first = decay[0], second = decay[CT - 1];
+                ow *= oct ? second : first;
+            } else {
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) {
+                    o[0][ct] *= decay[ct];
+                    o[1][ct] *= decay[ct];
+                }
             }
             probs(j - 1);
             __syncthreads();
         }
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) l[ct] += total_prev[ct];
+        if constexpr (kWide) {
+            // step s takes the 16 tokens of wave s: lane (column lane % 32, half lane / 32) 8 of them, P as
+            // published, V in one 8-byte read of dimension 32 wave + lane % 32. Two MFMAs of 32 cycles a
+            // step leave issue slots for its eight conversions (1000 + 476 keys and rows 40.3 -> 38.3
+            // us against 16x16 tiles)
+            const int half = lane >> 5, d = 32 * wave + (lane & 31);
+            half8 ps[2][2];
+            uint2 w8[2];
+            auto read = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
-        for (int s = 0; s < kDecodeWaves / 2; s++) {
-            const int src = 2 * s + (qq >> 1);
-            half8 ps[CT][2];
+                for (int hl = 0; hl < 2; hl++) ps[s & 1][hl] = *reinterpret_cast<const half8 *>(&pshare[slot][oct][hl][s][n][2 * half]);
+                w8[s & 1] = reinterpret_cast<const uint2 *>(&vbuf[slot][d][s ^ ((d >> 1) & 7)])[half];
+            };
+            read(0);
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++)
-#pragma unroll
-                for (int hl = 0; hl < 2; hl++)
-                    ps[ct][hl] = *reinterpret_cast<const half8 *>(&pshare[slot][ct][hl][src][n][2 * (qq & 1)]);
-#pragma unroll
-            for (int dt = 0; dt < 2; dt++) {
-                const int d = 16 * (2 * wave + dt) + n;
-                const uint2 w8 = reinterpret_cast<const uint2 *>(&vbuf[slot][d][src ^ ((d >> 1) & 7)])[qq & 1];
+            for (int s = 0; s < kDecodeWaves; s++) {
+                if (s + 1 < kDecodeWaves) read(s + 1);
                 uint32_t h0, h1, h2, h3;
-                i8x8_to_f16_sdwa(w8.x, w8.y, h0, h1, h2, h3);
+                i8x8_to_f16_sdwa(w8[s & 1].x, w8[s & 1].y, h0, h1, h2, h3);
                 const half8 va8 = __builtin_bit_cast(half8, make_uint4(h0, h1, h2, h3));
 #pragma unroll
-                for (int ct = 0; ct < CT; ct++) {
-                    o[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va8, ps[ct][0], o[dt][ct], 0, 0, 0);
-                    o[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va8, ps[ct][1], o[dt][ct], 0, 0, 0);
+                for (int hl = 0; hl < 2; hl++) ow = __builtin_amdgcn_mfma_f32_32x32x16_f16(va8, ps[s & 1][hl], ow, 0, 0, 0);
+            }
+        } else {
+            // step s takes the 32 tokens of waves 2s and 2s + 1, its operands read a step ahead
+            half8 ps[2][CT][2];
+            uint2 w8[2][2];
+            auto read = [&](int s) __attribute__((always_inline)) {
+                const int src = 2 * s + (qq >> 1);
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+                    for (int hl = 0; hl < 2; hl++)
+                        ps[s & 1][ct][hl] = *reinterpret_cast<const half8 *>(&pshare[slot][ct][hl][src][n][2 * (qq & 1)]);
+#pragma unroll
+                for (int dt = 0; dt < 2; dt++) {
+                    const int d = 16 * (2 * wave + dt) + n;
+                    w8[s & 1][dt] = reinterpret_cast<const uint2 *>(&vbuf[slot][d][src ^ ((d >> 1) & 7)])[qq & 1];
+                }
+            };
+            read(0);
+#pragma unroll
+            for (int s = 0; s < kDecodeWaves / 2; s++) {
+                if (s + 1 < kDecodeWaves / 2) read(s + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int dt = 0; dt < 2; dt++) {
+                    uint32_t h0, h1, h2, h3;
+                    i8x8_to_f16_sdwa(w8[s & 1][dt].x, w8[s & 1][dt].y, h0, h1, h2, h3);
+                    const half8 va8 = __builtin_bit_cast(half8, make_uint4(h0, h1, h2, h3));
+#pragma unroll
+                    for (int hl = 0; hl < 2; hl++)
+#pragma unroll
+                        for (int ct = 0; ct < CT; ct++)
+                            o[dt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va8, ps[s & 1][ct][hl], o[dt][ct], 0, 0, 0);
                 }
             }
         }
     };
-    auto phase = [&](uint32_t j, auto odd, bool store_knext, bool load_v2, bool load_k3) __attribute__((always_inline)) {
-        VRegs &rv = decltype(odd)::value ? vb : va;
-        KRegs &rk = decltype(odd)::value ? ka : kb;
+    for (uint32_t j = 0; j < nchunks; j++) {
+        v4i kop[4];   // chunk j's K operands, this wave's own rows: read ahead of chunk j - 1's end
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) kop[jj] = __builtin_bit_cast(v4i, kbuf[wave][n][(4 * jj + qq) ^ n]);
         if (j > 0) finish(j);
         {
-            v4i acc[CT][3];
+            v4i acc[CT][3], q3[2][CT];
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++)
+            for (int ct = 0; ct < CT; ct++) {
 #pragma unroll
                 for (int part = 0; part < 3; part++) acc[ct][part] = v4i{0, 0, 0, 0};
+                q3[0][ct] = q3lds[ct][0][16 * qq + (n ^ qq)];
+            }
 #pragma unroll
             for (int jj = 0; jj < 4; jj++) {
-                const v4i kop = __builtin_bit_cast(v4i, kbuf[wave][n][(4 * jj + qq) ^ n]);
-                const int slot = 16 * qq + (n ^ (4 * jj + qq));
+                if (jj < 3) {
+#pragma unroll
+                    for (int ct = 0; ct < CT; ct++) q3[(jj + 1) & 1][ct] = q3lds[ct][jj + 1][16 * qq + (n ^ (4 * jj + 4 + qq))];
+                }
 #pragma unroll
                 for (int ct = 0; ct < CT; ct++) {
-                    acc[ct][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, qi[ct][0][jj], acc[ct][0], 0, 0, 0);
-                    acc[ct][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, qi[ct][1][jj], acc[ct][1], 0, 0, 0);
-                    acc[ct][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop, q3lds[ct][jj][slot], acc[ct][2], 0, 0, 0);
+                    acc[ct][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[jj], qi[ct][0][jj], acc[ct][0], 0, 0, 0);
+                    acc[ct][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[jj], qi[ct][1][jj], acc[ct][1], 0, 0, 0);
                 }
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++)
+                    acc[ct][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kop[jj], q3[jj & 1][ct], acc[ct][2], 0, 0, 0);
             }
             const int local0 = (int)(j * kChunk) + 16 * wave + 4 * qq;   // token offset inside the split
             const uint32_t t0 = begin + (uint32_t)local0;
@@ -1545,31 +1600,14 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
             if (j > 0) probs(j);
         }
         store_v(j & 1, rv);
-        if (load_v2) load_v(rv, j + 2);
-        if (store_knext) store_k(rk);
-        if (load_k3) load_k(rk, j + 3);
-        __syncthreads();
-    };
-    uint32_t c = 0;
-    for (; c + 4 < nchunks; c += 2) {
-        phase(c, std::false_type{}, true, true, true);
-        phase(c + 1, std::true_type{}, true, true, true);
-    }
-    phase(c, std::false_type{}, c + 1 < nchunks, c + 2 < nchunks, c + 3 < nchunks);
-    uint32_t last_phase = c + 1;
-    if (c + 1 < nchunks) {
-        phase(c + 1, std::true_type{}, c + 2 < nchunks, c + 3 < nchunks, false);
-        last_phase = c + 2;
-        if (c + 2 < nchunks) {
-            phase(c + 2, std::false_type{}, c + 3 < nchunks, false, false);
-            last_phase = c + 3;
-            if (c + 3 < nchunks) {
-                phase(c + 3, std::true_type{}, false, false, false);
-                last_phase = c + 4;
-            }
+        if (j + 1 < nchunks) {
+            load_v(rv, j + 1);
+            store_k(rk);
         }
+        if (j + 2 < nchunks) load_k(rk, j + 2);
+        __syncthreads();
     }
-    finish(last_phase);
+    finish(nchunks);
 
     // ---- O^T[d][n] times the column's V scale reference, l over the lanes and waves
 #pragma unroll
@@ -1577,16 +1615,30 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         const float lt = xl_sum32(xl_sum16(l[ct]));
         if (qq == 0) wave_l[ct][wave][n] = lt;
     }
+    // the lane's quads of O, four dimensions of one column each: tile, first dimension, values
+    constexpr int kQuads = kWide ? 4 : 2 * CT;
+    auto quad_tile = [&](int u) __attribute__((always_inline)) { return kWide ? oct : u / 2; };
+    auto quad_dim = [&](int u) __attribute__((always_inline)) {
+        return 32 * wave + (kWide ? 8 * u + 4 * (lane >> 5) : 16 * (u % 2) + 4 * qq);
+    };
+    auto quad = [&](int u) __attribute__((always_inline)) {
+        float v;
+        floatx4 x;
+        if constexpr (kWide) {
+            const float first = vref[0], second = vref[CT - 1];
+            v = oct ? second : first;
+            x = floatx4{ow[4 * u], ow[4 * u + 1], ow[4 * u + 2], ow[4 * u + 3]};
+        } else {
+            v = vref[u / 2];
+            x = o[u % 2][u / 2];
+        }
+        return make_float4(x[0] * v, x[1] * v, x[2] * v, x[3] * v);
+    };
     if (p.splits > 1) {   // the partials' O needs no other wave's l
 #pragma unroll
-        for (int ct = 0; ct < CT; ct++) {
-            const uint32_t ri = 2 * ct + (n >> 3);
-            if (ri >= nr) continue;
-            float *part = part_of(ri) + head * 256 + 32 * wave + 4 * qq;
-#pragma unroll
-            for (int dt = 0; dt < 2; dt++)
-                *reinterpret_cast<float4 *>(part + 16 * dt) = make_float4(o[dt][ct][0] * vref[ct], o[dt][ct][1] * vref[ct],
-                                                                          o[dt][ct][2] * vref[ct], o[dt][ct][3] * vref[ct]);
+        for (int u = 0; u < kQuads; u++) {
+            const uint32_t ri = 2 * quad_tile(u) + (n >> 3);
+            if (ri < nr) *reinterpret_cast<float4 *>(part_of(ri) + head * 256 + quad_dim(u)) = quad(u);
         }
         __syncthreads();
         if (wave == 0 && qq == 0) {
@@ -1606,30 +1658,29 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     }
     // gate and y need only 4-byte alignment; all gate loads go out before the first store (the
     // compiler cannot tell y from gate)
-    float gate[CT][2][4];
+    float gate[kQuads][4];
+    auto out_at = [&](int u) __attribute__((always_inline)) {
+        const uint32_t row = r0 + min((uint32_t)(2 * quad_tile(u) + (n >> 3)), nr - 1);
+        return ((size_t)row * 16 + g * 8 + head) * 256 + quad_dim(u);
+    };
 #pragma unroll
-    for (int ct = 0; ct < CT; ct++) {
-        const uint32_t row = r0 + min((uint32_t)(2 * ct + (n >> 3)), nr - 1);
-        const float *at = p.gate + ((size_t)row * 16 + g * 8 + head) * 256 + 32 * wave + 4 * qq;
+    for (int u = 0; u < kQuads; u++)
 #pragma unroll
-        for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) gate[ct][dt][e] = at[16 * dt + e];
-    }
+        for (int e = 0; e < 4; e++) gate[u][e] = p.gate[out_at(u) + e];
     __syncthreads();
 #pragma unroll
-    for (int ct = 0; ct < CT; ct++) {
-        const uint32_t ri = 2 * ct + (n >> 3);
+    for (int u = 0; u < kQuads; u++) {
         float lw = 0.0f;
 #pragma unroll
-        for (int w = 0; w < kDecodeWaves; w++) lw += wave_l[ct][w][n];
-        if (ri >= nr) continue;
+        for (int w = 0; w < kDecodeWaves; w++) lw += wave_l[quad_tile(u)][w][n];
+        if ((uint32_t)(2 * quad_tile(u) + (n >> 3)) >= nr) continue;
         const float inv = 1.0f / lw;
-        float *at = p.y + ((size_t)(r0 + ri) * 16 + g * 8 + head) * 256 + 32 * wave + 4 * qq;
-#pragma unroll
-        for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) at[16 * dt + e] = o[dt][ct][e] * vref[ct] * inv * sigmoidf(gate[ct][dt][e]);
+        const float4 x = quad(u);
+        float *at = p.y + out_at(u);
+        at[0] = x.x * inv * sigmoidf(gate[u][0]);
+        at[1] = x.y * inv * sigmoidf(gate[u][1]);
+        at[2] = x.z * inv * sigmoidf(gate[u][2]);
+        at[3] = x.w * inv * sigmoidf(gate[u][3]);
     }
 }
 

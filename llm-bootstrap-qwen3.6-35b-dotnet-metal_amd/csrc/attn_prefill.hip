@@ -1172,7 +1172,7 @@ const char *launch_prefill(Context &c, const View *b, const boot_kernel_args &a,
     // * up to 64 rows and 2^19 row-key pairs: the multi-row kernel, which reads the keys once per four
     //   rows: (8000, 16) 26.7 / 20.9 / 41.0, (30000, 12) - / 29.2 / 50.9, (12000, 40) - / 38.2 / 40.9,
     //   (8000, 64) - / 39.7 / 39.3 us;
-    // * up to 512 rows in one split, 8 us and 2.4 us per 128 keys: (0, 256) 13.6 / 24.2, (600, 400)
+    // * up to 512 rows in one split, 8 us and 2.5 us per 128 keys: (0, 256) 13.6 / 24.2, (600, 400)
     //   28.7 / 35.5, (700, 200) 27.0 / 30.9, (1100, 256) 34.4 / 33.3, (1024, 512) 39.8 / 38.9 us.
     if (int8 && rows <= 512) {
         const uint64_t chunks = (keys + 127) / 128, work = rows * keys;
