@@ -54,6 +54,9 @@ constexpr int kTileRows = 256;             // logical rows per work-group (32 to
 // rows. FP16 rows, the common case, are as compact as a plain FP16 partial.
 constexpr size_t kPartialRegion = (size_t)kTileRows * 512;
 constexpr size_t kPartialBytes = 2 * kPartialRegion + 3 * kTileRows * 4;
+// Partials that the no-allocation dispatch's 72 MiB scratch holds. A launch takes more only with splits
+// of 256 keys and more (from 1505 rows).
+constexpr uint64_t kMostPartials = 284;
 // A row's partial is FP16 when its outputs are at most this large (FP16's relative 2^-12 of 4 is
 // 9.8e-4), FP32 otherwise.
 constexpr float kNarrowPartial = 4.0f;
@@ -1201,10 +1204,20 @@ const char *launch_prefill(Context &c, const View *b, const boot_kernel_args &a,
     // gain down to a tile or two per split: attention + combine, same box, (256 rows, no history)
     // 1 split 37.9, 2 25.5, 8 22.9 us; (512 rows after 512 keys) 4 splits 39.8, 8 33.7; (476 after
     // 1024) 5 splits 44.6, 8 38.1, 10 (two rounds) 55.8; (300 after 2100) 9 splits 43.7, 12 40.3, 16
-    // (two rounds) 56.2 us. The partials stay below one per CU (64.8 MiB on 256 CUs).
+    // (two rounds) 56.2 us.
     const uint64_t base_blocks = 2ull * p.tiles;
     const uint64_t round = (uint64_t)std::max(1, context_cus(c));
     uint64_t splits = std::max<uint64_t>(1, std::min<uint64_t>(round / base_blocks, keys / kW64Keys));
+    // One split more, into a second round, where the causal range leaves blocks short enough to make
+    // room for it: against one round's full block, the mean work of a CU and half a block. 1500 rows
+    // after 1500 keys 118 us in two splits (188 blocks), 102 in three (282); after 20000 593 and 732;
+    // 1100 rows alone 52.9 in three (210), 63.4 in four (280).
+    auto block_us = [&](uint64_t n) { return 17 + 2 * (((keys + n - 1) / n + kW64Keys - 1) / kW64Keys); };
+    const uint64_t more = splits + 1, blocks_more = base_blocks * more;
+    const uint64_t mean = (base_blocks * (a.pos + (rows + 32) / 2) / (kW64Keys / 2) + 17 * blocks_more) / round;
+    if (splits * base_blocks < round && blocks_more > round && more <= keys / kW64Keys && mean + block_us(more) / 2 < block_us(splits) &&
+        (blocks_more <= kMostPartials || more <= keys / 256))
+        splits = more;
     if (keys < 512) splits = 1;   // (FP16 storage only) few keys: the partials' FP16 rounding would show
     uint64_t split_keys = (keys + splits - 1) / splits;
     split_keys = (split_keys + kW64Keys - 1) / kW64Keys * kW64Keys;

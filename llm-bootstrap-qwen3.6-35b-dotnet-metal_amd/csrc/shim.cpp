@@ -26,8 +26,8 @@
 namespace boot {
 
 // Split-K scratch of boot_dispatch_noalloc (the attention kernels' per-split partials): 72 MiB,
-// enough for prefill chunks of any size on 256 CUs (at most one partial of 265,216 bytes per CU)
-// and for single-token decode up to the 262144 window (about 2 MiB). Each
+// enough for prefill chunks of up to 1504 rows and of 2048 rows on 256 CUs (at most 284 partials
+// of 265,216 bytes) and for single-token decode up to the 262144 window (about 2 MiB). Each
 // device holds its own copy until the process ends; the host reaches it only through the
 // address kept per device below.
 constexpr uint64_t kStaticScratchBytes = 72ull << 20;
