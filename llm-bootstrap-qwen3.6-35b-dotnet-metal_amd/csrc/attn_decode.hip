@@ -443,8 +443,6 @@ struct DecodeParams {
     const _Float16 *qh;          // prefill chunks routed here: the grouped FP16 query [2][rows][8][256]
 };
 
-// sigmoid(x) = 1 / (1 + 2^(-x log2(e))) with the hardware exponential and reciprocal (about an ulp
-// each), as the prefill kernels compute it
 // x of lane l ^ 16 (v_permlane16_swap) and of lane l ^ 32 (v_permlane32_swap) added or maxed in:
 // with both operands holding x, every lane ends with its own value in one register and its
 // partner's in the other; the no-ops cover the cross-lane move's wait states. Registers, not an
@@ -486,6 +484,8 @@ __device__ inline void wave_allmax(float (&x)[N]) {
     for (int i = 0; i < N; i++) x[i] = xl_max32(xl_max16(x[i]));
 }
 
+// sigmoid(x) = 1 / (1 + 2^(-x log2(e))) with the hardware exponential and reciprocal (about an ulp
+// each), as the prefill kernels compute it
 __device__ inline float sigmoidf(float x) {
     return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-x * 1.4426950408889634f));
 }
@@ -1794,13 +1794,17 @@ namespace {
 
 // Split geometry shared by both decode entry points: whole 128-token chunks per split, chosen so
 // that the grid (splits x 2 groups x rows, one work-group per CU) fits the CUs in one round (a
-// second, nearly empty round would double the time), at most kMaxSplitTokens per split.
+// second, nearly empty round would double the time), at most kMaxSplitTokens per split. Two chunks
+// stay in one split: the second chunk takes less than the combine's launch, which falls away (ten
+// layers' token after 128 to 255 tokens 115-121 us in two splits, 101-106 in one); three chunks
+// measure the same either way (119-121 us after 256 to 383 tokens).
 template <bool kHalfQ = false>
 const char *decode_launch(Context &c, DecodeParams &d, uint64_t rows, uint64_t length) {
     const uint64_t total_chunks = (length + kChunk - 1) / kChunk;
     const uint64_t slots = std::max<uint64_t>(1, (uint64_t)std::max(1, context_cus(c)) / (2 * rows));
     uint64_t split_chunks = (total_chunks + slots - 1) / slots;
     split_chunks = std::min<uint64_t>(split_chunks, (uint64_t)(kMaxSplitTokens / kChunk));
+    if (total_chunks == 2) split_chunks = 2;
     const uint64_t splits = (total_chunks + split_chunks - 1) / split_chunks;
     BOOT_REQUIRE(splits <= kMaxDecodeSplits, "too many decode splits");
     d.rows = (uint32_t)rows;
