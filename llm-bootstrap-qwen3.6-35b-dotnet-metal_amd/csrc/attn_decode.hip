@@ -558,6 +558,10 @@ __device__ __attribute__((always_inline)) inline void query_parts(const float4 &
                   __builtin_amdgcn_perm(t[part][3], t[part][2], 0x04000c0cu);
 }
 
+// The least reference of a split's V scales: 128 over it is FP32's 2^126. Smaller scales (vectors below
+// 1.9e-34) give operands below the full 2^7 instead of an infinite factor.
+constexpr float kLeastVScale = 0x1p-119f;
+
 // One chunk of one KV group in flight, K and V in separate register sets (K is staged
 // one chunk ahead of V): thread t holds K rows t / 16 + 32 i (16 bytes at 16 (t % 16))
 // and V page-row segments t / 8 + 64 i (16 bytes at 16 (t % 8)), i < 4: every load
@@ -866,7 +870,8 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     for (int w = 1; w < kDecodeWaves; w++) vs_ref = fmaxf(vs_ref, red[w]);
     // operands up to 2^8 times 2^7 stay below FP16's 65504; the factor keeps their lo parts out of its
     // subnormals
-    const float vs_inv = vs_ref > 0.0f ? 128.0f / vs_ref : 0.0f;
+    vs_ref = fmaxf(vs_ref, kLeastVScale);
+    const float vs_inv = 128.0f / vs_ref;
     vs_ref *= 1.0f / 128.0f;
     const float qsc = qmax[head] * (1.0f / 127.0f);   // s_q of the lane's head
     v4i qi[4], q3i[4];
@@ -1364,7 +1369,8 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         vref[ct] = n >= 8 ? odd : even;
         // operands up to 2^8 times 2^7 stay below FP16's 65504; the factor keeps their lo parts out of
         // its subnormals
-        vinv[ct] = vref[ct] > 0.0f ? 128.0f / vref[ct] : 0.0f;
+        vref[ct] = fmaxf(vref[ct], kLeastVScale);
+        vinv[ct] = 128.0f / vref[ct];
         vref[ct] *= 1.0f / 128.0f;
         qsc[ct] = qmax[ct][n] * (1.0f / 127.0f);
         row_end[ct] = first_end + min((uint32_t)(2 * ct + (n >> 3)), nr - 1);
@@ -1405,18 +1411,25 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         for (int ct = 0; ct < CT; ct++) {
             // m = -inf only in a column without a score yet
             const float refc = fmaxf(m[ct], -3.0e38f);
-            float arg[4], scaled[4];
+            float arg[4], vf[4], scaled[4];   // vf: the operands' V factors
 #pragma unroll
-            for (int r = 0; r < 4; r++) arg[r] = fmaf(dot_prev[ct][r], qsc[ct] * ksr[r], -refc);
-            if (edge)   // uniform
+            for (int r = 0; r < 4; r++) {
+                arg[r] = fmaf(dot_prev[ct][r], qsc[ct] * ksr[r], -refc);
+                vf[r] = vsr[r] * vinv[ct];
+            }
+            if (edge)   // uniform. A token the row does not see may exceed vref by any factor: its vf too is 0
 #pragma unroll
-                for (int r = 0; r < 4; r++) arg[r] = t0 + r < row_end[ct] ? arg[r] : -INFINITY;
+                for (int r = 0; r < 4; r++) {
+                    const bool seen = t0 + r < row_end[ct];
+                    arg[r] = seen ? arg[r] : -INFINITY;
+                    vf[r] = seen ? vf[r] : 0.0f;
+                }
             float total = 0.0f;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const float prob = __builtin_amdgcn_exp2f(arg[r]);   // 0 for masked tokens
                 total += prob;
-                scaled[r] = prob * (vsr[r] * vinv[ct]);
+                scaled[r] = prob * vf[r];
                 // one rounded FP32 value: else the operand's hi is the exact product rounded once
                 // (v_fma_mixlo_f16) and the hi that lo completes the rounded product rounded again,
                 // which differ by 2^-10 in rare near-ties
