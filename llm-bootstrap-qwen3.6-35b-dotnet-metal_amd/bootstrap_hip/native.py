@@ -12,7 +12,6 @@ There is no CPU fallback: if the library or a gfx950 device is missing, construc
 from __future__ import annotations
 
 import ctypes
-import operator
 import os
 import struct
 import weakref
@@ -246,17 +245,18 @@ class Device:
                     offsets.append(b.offset)
         try:
             pack = _PACKERS[count]
-            handles = pack(*handles)
-            if offsets is not None:
-                offsets = pack(*offsets)
+            handles, offsets = pack(*handles), None if offsets is None else pack(*offsets)
         except (struct.error, IndexError):   # more bindings; offsets outside 64 bits wrap as in C
-            pack = struct.Struct(f"{count}Q").pack
-            handles = handles if isinstance(handles, bytes) else pack(*handles)
-            if offsets is not None:
-                offsets = pack(*[operator.index(v) & 0xFFFFFFFFFFFFFFFF for v in offsets])
-        # (called without argument types: every argument is already the C type it is passed as)
-        if self._entries[noalloc](self._context, kernel.encode(), handles, offsets, count, _byref(args), _ARGS_BYTES,
-                                  threads_x, threads_y, 1, group, 1, 1, None, _NO_OFFSET) == 0:
+            handles = (ctypes.c_void_p * max(count, 1))(*handles)
+            offsets = (ctypes.c_uint64 * max(count, 1))(*(offsets or ()))
+        # plain ints of 32 bits pass as they are; anything else (NumPy integers, wider ints) by the
+        # declared argument types, which convert or refuse it
+        if type(threads_x) is type(threads_y) is type(group) is int and (threads_x | threads_y | group) >> 32 == 0:
+            entry = self._entries[1 if noalloc else 0]
+        else:
+            entry = self.lib.boot_dispatch_noalloc if noalloc else self.lib.boot_dispatch
+        if entry(self._context, kernel.encode(), handles, offsets, count, _byref(args), _ARGS_BYTES,
+                 threads_x, threads_y, 1, group, 1, 1, None, _NO_OFFSET) == 0:
             self._check(0)
 
     def close(self) -> None:

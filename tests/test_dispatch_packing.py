@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from bootstrap_hip import HipError, KernelArgs
-from bootstrap_hip.native import Binding, Device, GpuBuffer
+from bootstrap_hip.native import SIGNATURES, Binding, Device, GpuBuffer
 
 
 @pytest.fixture
@@ -67,3 +67,61 @@ def test_a_failed_dispatch_raises_with_the_context_error(recorder):
     recorder.lib = Lib
     with pytest.raises(HipError, match="no such kernel"):
         recorder.dispatch("k", KernelArgs(), 64, 256)
+
+
+@pytest.fixture
+def native():
+    """A device whose entries are C function pointers (into Python), typed and untyped as the library's."""
+    device = Device.__new__(Device)
+    device.handle, device._context, device.calls = 0x1000, ctypes.c_void_p(0x1000), []
+
+    class Untyped(ctypes._CFuncPtr):
+        _flags_, _restype_ = ctypes._FUNCFLAG_CDECL, ctypes.c_int
+
+    class Lib:
+        pass
+    device.lib, device.kept, entries = Lib, [], []
+    for name in ("boot_dispatch", "boot_dispatch_noalloc"):
+        result, types = SIGNATURES[name]
+        typed = ctypes.CFUNCTYPE(result, *types)(lambda *a, name=name: device.calls.append((name, a)) or 1)
+        device.kept.append(typed)
+        pointer = Untyped(ctypes.cast(typed, ctypes.c_void_p).value)
+        entries.append(pointer)
+        bound = Untyped(ctypes.cast(typed, ctypes.c_void_p).value)
+        bound.argtypes = types
+        setattr(Lib, name, staticmethod(bound))
+    device._entries = tuple(entries)
+    yield device
+    device.handle = 0
+
+
+@pytest.mark.parametrize("value,expected", [
+    (64, 64), (np.int64(64), 64), (np.uint32(64), 64), (np.int32(64), 64), (True, 1), (0, 0), (2 ** 32 - 1, 2 ** 32 - 1),
+    (-1, 2 ** 32 - 1), (2 ** 32 + 64, 64), (2 ** 70 + 64, 64), (ctypes.c_uint32(64), 64)])
+def test_thread_counts_convert_as_uint32(native, value, expected):
+    buffer = GpuBuffer(native, 0x7f0000000000, 1 << 20)
+    native.dispatch("k", KernelArgs(), value, 256, buffer)
+    native.dispatch("k", KernelArgs(), 64, value, buffer)
+    native.dispatch2d("k", KernelArgs(), 64, value, 256, buffer.at(8), noalloc=True)
+    assert [name for name, _ in native.calls] == ["boot_dispatch", "boot_dispatch", "boot_dispatch_noalloc"]
+    assert [a[7:13] for _, a in native.calls] == [(expected, 1, 1, 256, 1, 1), (64, 1, 1, expected, 1, 1),
+                                                  (64, expected, 1, 256, 1, 1)]
+    assert all(a[0] == 0x1000 and a[1] == b"k" and a[4] == 1 and a[6] == 64 and a[13] is None and a[14] == 0
+               for _, a in native.calls)
+
+
+@pytest.mark.parametrize("value", [1.5, "64", None, ctypes.c_double(64.0), b"64"])
+def test_thread_counts_of_other_types_are_refused(native, value):
+    with pytest.raises(ctypes.ArgumentError):
+        native.dispatch("k", KernelArgs(), value, 256)
+    with pytest.raises(ctypes.ArgumentError):
+        native.dispatch2d("k", KernelArgs(), 64, 1, value)
+    assert native.calls == []
+
+
+@pytest.mark.parametrize("noalloc,name", [(False, "boot_dispatch"), (None, "boot_dispatch"), (0, "boot_dispatch"),
+                                          (True, "boot_dispatch_noalloc"), (2, "boot_dispatch_noalloc"),
+                                          (np.bool_(True), "boot_dispatch_noalloc"), ("yes", "boot_dispatch_noalloc")])
+def test_noalloc_takes_truth_values(native, noalloc, name):
+    native.dispatch("k", KernelArgs(), 64, 256, noalloc=noalloc)
+    assert [called for called, _ in native.calls] == [name]
