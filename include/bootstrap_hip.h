@@ -110,7 +110,8 @@ int boot_read(void *ctx, void *buf, uint64_t offset, void *host, uint64_t bytes)
  * context workspace; it calls no hipMalloc/hipFree or other allocating routine and records no
  * timing sample. Requests larger than 72 MiB are rejected (0, with the size in boot_error) before
  * any launch; 72 MiB covers prefill chunks of up to 1504 rows and of 2048 rows on 256 CUs,
- * single-token decode up to the 262144 window, and the scalar reader for 8 rows up to 262144
+ * single-token decode up to the 262144 window, verify blocks of 64 rows up to 65536 keys and of 35
+ * rows up to the window, and the scalar reader for 8 rows up to 262144
  * keys (values partials: rows x 2 x keys / 512 x 8 KiB, 64 MiB there). One GPU has one array: the first split-K call of a command claims it
  * for that context until the command's boot_end, and a split-K call of another context meanwhile
  * fails (0, "held by another context's command") instead of racing; calls in one context's

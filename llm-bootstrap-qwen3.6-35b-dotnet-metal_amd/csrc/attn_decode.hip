@@ -1950,9 +1950,31 @@ const char *launch_verify_int8(Context &c, const View *b, int count, const boot_
     };
     static_assert(kNearChunks <= kNearSlots * (kMaxSplitTokens / kChunk) &&
                       262144 / kChunk <= kFarSlots * (kMaxSplitTokens / kChunk), "a split's scales exceed the LDS");
-    for (uint64_t first = 0; first < rows;) {
+    // one past the last row of the launch that starts with row `first`, and that launch's splits
+    auto launch_end = [&](uint64_t first) {
         uint64_t next = first + 1;
         while (next < rows && split_of(next) == split_of(first)) next++;
+        return next;
+    };
+    auto splits_of = [&](uint64_t first, uint64_t next) {
+        const uint32_t per = split_of(first);
+        return (chunks_of(next - 1) + per - 1) / per;
+    };
+    // The scratch of the largest launch, before the first one: y may be q, so a request refused after a
+    // launch would leave some queries overwritten.
+    uint64_t scratch = 0;
+    for (uint64_t first = 0, next; first < rows; first = next) {
+        next = launch_end(first);
+        const uint64_t splits = splits_of(first, next);
+        if (splits > 1) scratch = std::max<uint64_t>(scratch, (next - first) * 2 * splits * kPartialFloats * sizeof(float));
+    }
+    float *partial = nullptr;
+    if (scratch) {
+        partial = (float *)context_workspace(c, scratch);
+        BOOT_REQUIRE(partial, "cannot allocate verify split workspace");
+    }
+    for (uint64_t first = 0, next; first < rows; first = next) {
+        next = launch_end(first);
         RowsParams d;
         d.qh = nullptr;
         d.q = (const float *)b[0].ptr + first * 4096;
@@ -1965,12 +1987,8 @@ const char *launch_verify_int8(Context &c, const View *b, int count, const boot_
         d.rows = (uint32_t)(next - first);
         d.pos = (uint32_t)(p.pos + first);
         d.split_chunks = split_of(first);
-        d.splits = (chunks_of(next - 1) + d.split_chunks - 1) / d.split_chunks;
-        d.partial = nullptr;
-        if (d.splits > 1) {
-            d.partial = (float *)context_workspace(c, (uint64_t)d.rows * 2 * d.splits * kPartialFloats * sizeof(float));
-            BOOT_REQUIRE(d.partial, "cannot allocate verify split workspace");
-        }
+        d.splits = splits_of(first, next);
+        d.partial = d.splits > 1 ? partial : nullptr;
         // one or two rows: half the columns and registers (1 row after 1500 keys 7.8 against 9.7 us)
         const bool narrow = d.rows <= 2;
         d.zs = narrow ? 1 : (d.rows + 3) / 4;
@@ -1983,7 +2001,6 @@ const char *launch_verify_int8(Context &c, const View *b, int count, const boot_
         if (d.splits > 1)
             launch_timed(c, "decode_combine_kernel", decode_combine_kernel, dim3(4, 16, d.rows), dim3(256),
                          (const float *)d.partial, d.gate, d.y, d.splits);
-        first = next;
     }
     return nullptr;
 }

@@ -162,3 +162,33 @@ def test_noalloc_refuses_beyond_the_static_scratch(device, oracle):
     device.end()
     for b in (k, v, q, gate, out, *scales):
         b.dispose()
+
+
+def test_noalloc_verify_is_refused_before_any_launch(device, oracle):
+    """64 verify rows across 65536 keys take two launches, and the second one's 54 rows x 2 x 103 split
+    partials of 8256 bytes (92 MB) exceed the scratch: refused with the query, which is also the
+    output, as it was; boot_dispatch then serves it (rows of both launches against FP64)."""
+    rows, history = 64, 65536 - 10
+    length = history + rows
+    host = host_cache(oracle, length, reference_kv(length))
+    cache = upload_cache(device, *host)
+    q, gate = oracle.fill_hash(rows * 4096, 17, 3), oracle.fill_hash(rows * 4096, 11, 1)
+    qb, gb = upload(device, q), upload(device, gate)
+    p = KernelArgs(M=rows, K=length, Position=history)
+    bindings = (qb, cache.kc, cache.vc, gb, qb, cache.ks, cache.vs)
+    device.begin()
+    with pytest.raises(HipError, match="static scratch"):
+        device.dispatch("attention_verify_int8", p, rows * 4096, 256, *bindings, noalloc=True)
+    device.end()
+    assert np.array_equal(qb.read(np.float32, rows * 4096), q), "a launch ran before the refusal"
+    device.begin()
+    device.dispatch("attention_verify_int8", p, rows * 4096, 256, *bindings)
+    device.end()
+    y = qb.read(np.float32, rows * 4096)
+    for r in (0, 9, 10, 63):
+        row = slice(r * 4096, (r + 1) * 4096)
+        ref = oracle.attention(q[row], *host, gate[row], 1, history + r, round_q_half=0)
+        assert rel_l2(y[row], ref) <= 5e-6
+    for b in (qb, gb):
+        b.dispose()
+    cache.dispose()
