@@ -1208,6 +1208,17 @@ const char *launch_prefill(Context &c, const View *b, const boot_kernel_args &a,
     const uint64_t base_blocks = 2ull * p.tiles;
     const uint64_t round = (uint64_t)std::max(1, context_cus(c));
     uint64_t splits = std::max<uint64_t>(1, std::min<uint64_t>(round / base_blocks, keys / kW64Keys));
+    // Few rows (many splits): the combine takes about 1.5 us per eight splits, which it reads one step
+    // after the other, a split 2 us per key tile: the tiles per split with the least sum. Attention +
+    // combine, one box, every CU taken / this rule / splits of 256 keys: FP16 storage, 16 rows after 2000
+    // keys 63 splits 32.1, 32 28.2, 7 38.2; 8 rows after 8000 126 45.7, 63 36.3, 28 40.2; after 16000 126
+    // 49.3, 72 45.7, 56 45.8; INT8, 65 rows after 2000 33 36.1, 22 34.6, 8 40.6 us.
+    const uint64_t key_tiles = (keys + kW64Keys - 1) / kW64Keys;
+    auto half_us = [&](uint64_t per) { return 4 * per + 3 * (((key_tiles + per - 1) / per + 7) / 8); };
+    uint64_t per_split = (key_tiles + splits - 1) / splits;
+    for (uint64_t per = per_split + 1; 4 * per < half_us(per_split); per++)
+        if (half_us(per) < half_us(per_split)) per_split = per;
+    splits = std::min(splits, (key_tiles + per_split - 1) / per_split);
     // One split more, into a second round, where the causal range leaves blocks short enough to make
     // room for it: against one round's full block, the mean work of a CU and half a block. 1500 rows
     // after 1500 keys 118 us in two splits (188 blocks), 102 in three (282); after 20000 593 and 732;
