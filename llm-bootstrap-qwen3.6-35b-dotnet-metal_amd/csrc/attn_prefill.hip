@@ -1219,16 +1219,34 @@ const char *launch_prefill(Context &c, const View *b, const boot_kernel_args &a,
     for (uint64_t per = per_split + 1; 4 * per < half_us(per_split); per++)
         if (half_us(per) < half_us(per_split)) per_split = per;
     splits = std::min(splits, (key_tiles + per_split - 1) / per_split);
-    // One split more, into a second round, where the causal range leaves blocks short enough to make
-    // room for it: against one round's full block, the mean work of a CU and half a block. 1500 rows
-    // after 1500 keys 118 us in two splits (188 blocks), 102 in three (282); after 20000 593 and 732;
-    // 1100 rows alone 52.9 in three (210), 63.4 in four (280).
+    // One split more, into a second round, where the causal range leaves blocks short enough to make room
+    // for it. Two bounds on its time, against one round's full block: the mean work of a CU and half a
+    // block (and 1 us per 32 blocks of the second round); and its longest chain: the second round's last
+    // block, the last row tile of the last split, starts when that split's first, shortest blocks have
+    // ended (up to 8 us more: the chain is the work of few CUs). Attention + combine, two splits / three:
+    // 1500 rows alone 88 / 87, after 1500 keys 129 / 114, after 2000 142 / 129, after 4000 200 / 199, after
+    // 6000 240 / 263, after 9000 310 / 368; 1450 rows after 2500 160 / 147; 1346 rows after 9000 302 / 357;
+    // 1600 rows after 250 keys 103 / 97, after 1000 122 / 126 us; 1100 rows alone 63 in three, 73 in four.
     auto block_us = [&](uint64_t n) { return 17 + 2 * (((keys + n - 1) / n + kW64Keys - 1) / kW64Keys); };
     const uint64_t more = splits + 1, blocks_more = base_blocks * more;
-    const uint64_t mean = (base_blocks * (a.pos + (rows + 32) / 2) / (kW64Keys / 2) + 17 * blocks_more) / round;
-    if (splits * base_blocks < round && blocks_more > round && more <= keys / kW64Keys && mean + block_us(more) / 2 < block_us(splits) &&
-        (blocks_more <= kMostPartials || more <= keys / 256))
-        splits = more;
+    if (splits * base_blocks < round && blocks_more > round && more <= keys / kW64Keys &&
+        (blocks_more <= kMostPartials || more <= keys / 256)) {
+        const uint64_t second = blocks_more - round;
+        const uint64_t mean = (base_blocks * (a.pos + (rows + 32) / 2) / (kW64Keys / 2) + 17 * blocks_more) / round;
+        // keys of the last split that row tile t sees; the tile whose block is the second round's last to
+        // start: the last split's blocks of both groups end in pairs up to the first round's share of the
+        // second group, then the first group's alone
+        const uint64_t before = splits * (((keys + more - 1) / more + kW64Keys - 1) / kW64Keys * kW64Keys);
+        auto seen = [&](uint64_t t) {
+            const uint64_t end = std::min<uint64_t>(keys, a.pos + kTileRows / 8 * (t + 1));
+            return end > before ? end - before : 0;
+        };
+        const uint64_t first_groups = (2 * splits + 1) * p.tiles, share = round > first_groups ? round - first_groups : 0;
+        const uint64_t at = second - 1 < 2 * share ? (second - 1) / 2 : second - 1 - share;
+        const uint64_t chain = 34 + (seen(std::min<uint64_t>(at, p.tiles - 1)) + seen(p.tiles - 1)) / (kW64Keys / 2);
+        const uint64_t full = block_us(splits), work = mean + block_us(more) / 2 + second / 32;
+        if (chain < full ? work <= full : work < full && chain < full + 8) splits = more;
+    }
     if (keys < 512) splits = 1;   // (FP16 storage only) few keys: the partials' FP16 rounding would show
     uint64_t split_keys = (keys + splits - 1) / splits;
     split_keys = (split_keys + kW64Keys - 1) / kW64Keys * kW64Keys;

@@ -21,3 +21,16 @@ def test_fp16_few_rows(device, oracle, history, rows):
 def test_int8_few_rows(device, oracle, history, rows):
     """Against FP64 at the bounds of the other prefill tests."""
     check_int8(device, oracle, history, rows)
+
+
+# more work-groups than CUs: 1500 and 1600 rows in three splits, 2200 in two; and next to them, in one
+# round, 1600 rows after a longer history and 1300 rows
+@pytest.mark.parametrize("history,rows", [(0, 1600), (1500, 1500), (2000, 1500), (0, 2200), (1000, 1600), (700, 1300)])
+def test_int8_second_round(device, oracle, history, rows):
+    """Against FP64 at the bounds of the other prefill tests."""
+    check_int8(device, oracle, history, rows)
+
+
+@pytest.mark.parametrize("history,rows", [(1000, 1450)])
+def test_fp16_second_round(device, oracle, history, rows):
+    check_fp16(device, oracle, history, rows, False)
