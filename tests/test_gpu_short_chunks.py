@@ -1,7 +1,8 @@
 """Prefill chunks over short key ranges and of few rows: the multi-row kernel (whole and partial row
 blocks, row blocks whose causal end lies chunks or splits before the range's end, one split and
-several), its edges against the decode kernel and the 256-row kernel, and that kernel's splits of one
-or two 32-key tiles, the last one ragged; decodes around two chunks of keys, which take one split."""
+several), its edges against the decode kernel and the 256-row kernel, and that kernel next to those
+edges (splits of two to seven 32-key tiles, the last one ragged); decodes around two chunks of keys,
+which take one split."""
 import numpy as np
 import pytest
 

@@ -1,14 +1,16 @@
 """Speculative verification over the INT8 cache, KV part of VerificationSelfTest
 (Verification.cs:105-139): a verify block of `width` candidate rows appended at the prompt end
-and read by the scalar reader (Prefill.cs:269-285), then committed at `retained` rows
+and attended by verify_attention_int8 (Prefill.cs:269-285: one dispatch up to 64 rows, the scalar
+reader beyond), then committed at `retained` rows
 (rollback = move the position back; the rejected KV stays in place, Verification.cs:5-8), must
 leave the same KV state and row outputs as verifying only the `retained` rows, and an unrelated
 continuation token must overwrite the rejected slot without reading anything stale."""
 import numpy as np
 import pytest
 
-from bootstrap_hip import Int8KvCache, engine
-from kvcase import upload
+from bootstrap_hip import Int8KvCache, KernelArgs, engine
+from kvcase import rel_l2, upload, upload_cache
+from test_gpu_attention import build_case
 
 pytestmark = pytest.mark.gpu
 
@@ -48,7 +50,7 @@ class Stream:
                 b.dispose()
 
 
-def run(device, cache, s, scores, prompt, verified, retained, workspace=engine.ATTENTION_WORKSPACE_FLOATS):
+def run(device, cache, s, scores, prompt, verified, retained, attend=engine.verify_attention_int8):
     """Reset, prefill the prompt, verify `verified` candidates, commit `retained`, continue once."""
     cache.reset()
     cache.ensure_capacity(prompt)
@@ -63,7 +65,7 @@ def run(device, cache, s, scores, prompt, verified, retained, workspace=engine.A
     for l, layer in enumerate(cache.layers):
         q, k, v, g = s.candidates[l]
         engine.append_rows(device, layer, q, k, v, s.verify[l], verified, prompt)
-        engine.verify_attention_int8(device, layer, s.verify[l], g, scores, verified, prompt, workspace)
+        attend(device, layer, s.verify[l], g, scores, verified, prompt)
     device.end()
     cache.position = prompt + verified
     rows = [s.verify[l].read(np.float32, verified * 4096).reshape(verified, 4096) for l in range(LAYERS)]
@@ -116,18 +118,56 @@ def test_verify_rollback_matches_accepted_prefix(device, prompt):
 
 
 def test_verify_slices_agree_with_one_slice(device):
-    """A score workspace too small for the whole block splits it into query slices
-    (Prefill.cs:273-276); each slice keeps its absolute position, so the rows are bitwise those
-    of one slice."""
+    """A block dispatched in query slices (Prefill.cs:273-276: 3 + 3 + 2 rows), each at its absolute
+    position, gives bitwise the rows of one dispatch."""
     prompt = 777
     s = Stream(device, prompt, seed=9)
     cache = Int8KvCache(device, context_window=4096, layers=LAYERS)
     scores = device.allocate(8 * 16 * (prompt + 9) * 4)
+    slices = engine.verify_slices(8, prompt, 3 * 16 * (prompt + 8))   # three rows' scores
+    assert slices == [(0, 3), (3, 3), (6, 2)]
+
+    def in_slices(device, layer, rotated, gate, scores, rows, position):
+        for first, count in slices:
+            p = KernelArgs(M=count, K=position + first + count, Position=position + first)
+            q, g = rotated.at(first * 16384), gate.at(first * 16384)
+            device.dispatch("attention_verify_int8", p, count * 4096, 256, q, layer.key, layer.value, g, q,
+                            layer.key_scale, layer.value_scale)
+
     whole = run(device, cache, s, scores, prompt, 8, 8)[0]
-    small = 3 * 16 * (prompt + 8)                                # three rows per slice: 3 + 3 + 2
-    assert engine.verify_slices(8, prompt, small) == [(0, 3), (3, 3), (6, 2)]
-    sliced = run(device, cache, s, scores, prompt, 8, 8, workspace=small)[0]
+    sliced = run(device, cache, s, scores, prompt, 8, 8, attend=in_slices)[0]
     for l in range(LAYERS):
         assert np.array_equal(whole[l], sliced[l])
     scores.dispose()
     s.dispose()
+
+
+def test_verify_beyond_64_rows_takes_the_reader_in_slices(device, oracle):
+    """A block of more rows than one attention_verify_int8 dispatch serves runs on the scalar reader, in
+    as many slices as the score workspace asks for: bitwise the rows of one slice, and within the
+    float32 reader's bound of FP64 (eight rounding steps of 2^-24 on base-2 scores up to about 2^3)."""
+    history, rows = 300, engine.VERIFY_ROWS + 6
+    length = history + rows
+    q, gate, host = build_case(oracle, history, rows)
+    device_cache = upload_cache(device, *host)
+    layer = engine.Int8KvLayer.__new__(engine.Int8KvLayer)
+    layer.key, layer.value = device_cache.kc, device_cache.vc
+    layer.key_scale, layer.value_scale = device_cache.ks, device_cache.vs
+    gb, scores = upload(device, gate), device.allocate(rows * 16 * length * 4)
+    got = []
+    for per in (rows, 32):
+        workspace = per * 16 * length
+        assert [n for _, n in engine.verify_slices(rows, history, workspace)] == ([rows] if per == rows else [32, 32, 6])
+        qb = upload(device, np.append(q, np.float32(np.nan)))
+        device.begin()
+        engine.verify_attention_int8(device, layer, qb, gb, scores, rows, history, workspace)
+        device.end()
+        got.append(qb.read(np.float32, rows * 4096 + 1))
+        qb.dispose()
+        assert np.isnan(got[-1][-1]), "output guard overwritten"
+    whole, sliced = (y[:-1] for y in got)
+    assert np.array_equal(whole.view(np.uint32), sliced.view(np.uint32))
+    assert rel_l2(whole, oracle.attention(q, *host, gate, rows, history, round_q_half=0)) <= 4e-6
+    for b in (gb, scores):
+        b.dispose()
+    device_cache.dispose()

@@ -1,5 +1,5 @@
 """boot_dispatch_noalloc (the entry point that allocates nothing) against boot_dispatch on the
-same inputs: split-K decode, prefill and the scalar reader on a fresh context, the no-allocation
+same inputs: split-K decode, prefill, verify blocks and the scalar reader on a fresh context, the no-allocation
 calls first (before the context has any workspace) with boot_allocated unchanged across each of
 them, two calls in a
 row with the second smaller, results bitwise equal and within the FP64 bar; sizes beyond the
@@ -86,15 +86,35 @@ def reader(device, q, gate, cache, rows, history, noalloc):
     return y[:-1]
 
 
+def verify(device, q, gate, cache, rows, history, noalloc):
+    """A verify block (attention_verify_int8), in place over its query as the engine dispatches it."""
+    qb, gb = upload(device, np.append(q, np.float32(np.nan))), upload(device, gate)
+    p = KernelArgs(M=rows, K=history + rows, Position=history)
+    before = device.allocated_bytes
+    device.begin()
+    device.dispatch("attention_verify_int8", p, rows * 4096, 256, qb, cache.kc, cache.vc, gb, qb, cache.ks, cache.vs,
+                    noalloc=noalloc)
+    device.end()
+    if noalloc:
+        assert device.allocated_bytes == before, "boot_dispatch_noalloc allocated device memory"
+    y = qb.read(np.float32, rows * 4096 + 1)
+    for b in (qb, gb):
+        b.dispose()
+    assert np.isnan(y[-1])
+    return y[:-1]
+
+
 @pytest.mark.parametrize("kind,cases", [
     ("decode", [(131071, 1), (4093, 7)]),        # 114 splits per group, then 6
-    ("prefill", [(30208, 512), (257, 33)]),      # 68 MB of partial slots, then a 33-row chunk (decode kernel, 3 splits)
+    ("prefill", [(30208, 512), (257, 33)]),      # 68 MB of partial slots, then a 33-row chunk (multi-row kernel, one split)
+    ("prefill", [(8128, 64), (1000, 16)]),       # multi-row kernel and decode kernel, 8 splits each
+    ("verify", [(65530, 12), (4093, 3)]),        # two launches (64 and 103 splits), then 33 splits
     ("reader", [(65528, 8), (4093, 3)]),         # 16 MB of values partials and 8-row softmax statistics, then 3 rows
 ])
 def test_noalloc_matches_dispatch(oracle, kind, cases):
     """A fresh context: every no-allocation call runs before the context has a workspace, so a
     path that fell back to (or grew) the workspace would show in boot_allocated."""
-    run = {"decode": decode, "prefill": prefill, "reader": reader}[kind]
+    run = {"decode": decode, "prefill": prefill, "verify": verify, "reader": reader}[kind]
     with Device() as device:
         prepared = []
         for history, rows in cases:
