@@ -351,10 +351,41 @@ def cpu_baseline(work: "PrefillWorkload", dec: "DecodeWorkload", y_last, runs: i
 
 # --------------------------------------------------------------------------- verify reader
 
+def verify_block(dec, rows: int = 8, runs: int = 5):
+    """The attention of a speculative verify block as the engine dispatches it (attention_verify_int8,
+    Prefill.cs:269-285) for `rows` draft rows at the end of config 4's cache (layer 0), kernel-exact,
+    mean of `runs` blocks."""
+    d = dec.device
+    layer = dec.cache.layers[0]
+    length = dec.pos0 + dec.steps
+    history = length - rows
+    out = d.allocate(rows * 16384)
+    p = KernelArgs(M=rows, K=length, Position=history)
+
+    def block():   # (not in place, as the engine has it: the query serves every run)
+        d.dispatch("attention_verify_int8", p, rows * 4096, 256, dec.q, layer.key, layer.value, dec.gate, out,
+                   layer.key_scale, layer.value_scale)
+
+    d.begin()
+    block()
+    d.end()
+    d.reset_wall_timing(kernels_exact=True)
+    d.begin()
+    for _ in range(runs):
+        block()
+    d.end()
+    ks = kernel_stats(d, ["rows_int8_kernel", "decode_combine_kernel"])
+    us = {n: round(ms / runs * 1000, 2) for n, (ms, _) in ks.items()}
+    out.dispose()
+    return {"history": history, "rows": rows, "kernel_us": us, "total_us": round(sum(us.values()), 2),
+            "kv_bytes": 1040 * length, "what": "one dispatch, four rows per work-group, and the splits' combine, "
+                                               "kernel-exact, one layer"}
+
+
 def verify_reader(dec, rows: int = 8, runs: int = 5):
-    """The scalar reader a speculative verify block runs (Prefill.cs:269-285, kernels.metal:147-166:
-    batch_attention_scores_int8, attention_softmax, batch_attention_values_int8) for `rows` draft
-    rows at the end of config 4's cache (layer 0), kernel-exact, mean of `runs` blocks."""
+    """The scalar reader (kernels.metal:147-166: batch_attention_scores_int8, attention_softmax,
+    batch_attention_values_int8), which serves direct callers and verify blocks of more than 64 rows,
+    for `rows` rows at the end of config 4's cache (layer 0), kernel-exact, mean of `runs` blocks."""
     d = dec.device
     layer = dec.cache.layers[0]
     length = dec.pos0 + dec.steps
@@ -605,7 +636,8 @@ def main():
             "traffic": measured_traffic("kv_store_int8 bulk 131072"),
             "bytes": bulk_bytes, "kernel_ms": round(bulk, 4)}
     if dec is not None:
-        log("verify reader: 8 rows at the end of config 4's cache")
+        log("verify block and scalar reader: 8 rows at the end of config 4's cache")
+        result["verify_block"] = verify_block(dec)
         result["verify_reader"] = verify_reader(dec)
     if not args.no_cpu_baseline:
         log("cpu baseline: the FP64 checker on configs 1, 2, a 131072 decode step and config 3's last chunk")
