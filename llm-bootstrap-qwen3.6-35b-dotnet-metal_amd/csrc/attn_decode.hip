@@ -1,10 +1,11 @@
-// Single-token (and 1-8 row verification) INT8 attention over the KV cache.
+// INT8 attention of single tokens, verify blocks and small prefill chunks over the KV cache.
 //
 // Three entry points:
 //   * the reference's three-kernel reader (kernels.metal:147-156,163-166):
 //     batch_attention_scores_int8 -> attention_softmax -> batch_attention_values_int8,
-//     FP32 scores in a caller buffer; serves serial decode and speculative
-//     verification unchanged (QwenEngine.cs:161-165, Prefill.cs:280-285).
+//     FP32 scores in a caller buffer; serves callers that dispatch it as the
+//     reference does (QwenEngine.cs:161-165, Prefill.cs:280-285) and verify blocks
+//     of more than 64 rows.
 //   * attention_decode_int8: one fused split-K pass that streams the INT8 K/V
 //     pages from HBM once, as whole K rows and whole 128-byte V page-row lines
 //     staged through LDS. Scores run on INT8 MFMA straight from the K codes:
@@ -13,10 +14,10 @@
 //     <= 6.1e-8 max|q| per element, below the FP32 reader's own summation error),
 //     in two MFMAs whose 16 columns are 8 heads x {q1, q2} and 8 heads x q3. PV runs on FP16 MFMA
 //     with V codes dequantized exactly in registers and the scaled
-//     probabilities p*vs[t]/vs_ref (vs_ref = the largest V scale of the split, so
-//     they lie in [0, 1]) split into FP16 hi + lo. Scales are applied to scores
-//     and probabilities as the reference does (score = dot * ks[t] / 16,
-//     P = p * vs[t]).
+//     probabilities 2^7 p*vs[t]/vs_ref (vs_ref = the largest V scale of the split; p is
+//     at most 2^8 against a lagging running maximum, so they lie in [0, 2^15]) split
+//     into FP16 hi + lo. Scales are applied to scores and probabilities as the
+//     reference does (score = dot * ks[t] / 16, P = p * vs[t]).
 //   * attention_verify_int8: the same arithmetic for the rows of a verify block, several
 //     rows per work-group (rows_int8_kernel).
 #include "common.h"
@@ -703,10 +704,10 @@ __device__ __attribute__((always_inline)) inline void patch_v(VRegs &r, int tid,
 // {q1, q2}, and a second product for q3), and turns them into probabilities in base 2 against a running reference
 // shared by the work-group; the waves exchange those P operands through LDS and wave w
 // accumulates O^T[d][n] += V^T[d][t] . Px[t][n] for dimensions 32w..32w+31 over all 128
-// tokens (16x16x32 FP16 MFMA), so no wave merge of O remains at the end. Px = p * vs /
+// tokens (16x16x32 FP16 MFMA), so no wave merge of O remains at the end. Px = 2^7 p * vs /
 // vs_ref split into FP16 hi + lo; vs_ref, the split's largest V scale, keeps Px below
-// 256 and multiplies the result once. Lane l holds MFMA column n = l % 16 and
-// token/k group qq = l / 16.
+// 2^15 (p <= 2^8, see below) and vs_ref / 2^7 multiplies the result once. Lane l holds MFMA
+// column n = l % 16 and token/k group qq = l / 16.
 // Up to about 16000 tokens a split is one chunk and the kernel one chunk's latency, most of it issue
 // (an instruction of all eight waves takes 8 cycles of a SIMD): the query's parts are built by a head
 // per wave, the prologue has one barrier (two for the work-group that appends), the first chunk's
@@ -731,8 +732,8 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     __shared__ float fresh_scale[2];
     // INT8 query operands [set][MFMA c][slot] (set 0: q1 | q2 columns, set 1: q3 in columns n < 8),
     // lane (n, qq)'s in slot 16 qq + (n ^ (4 c + qq)) as in rows_int8_kernel, built once and read
-    // into registers before the chunk loop. They sit in the V half of chunk buffer 1, which is first written in phase 1, after the barrier that ends phase 0: by then every
-    // wave has read its operands.
+    // into registers before the chunk loop. They sit in the V half of chunk buffer 1, which is first
+    // written in phase 1, after the barrier that ends phase 0: by then every wave has read its operands.
     v4i(*qlds)[4][64] = reinterpret_cast<v4i(*)[4][64]>(&bufs[1].v[0][0]);
     static_assert(2 * 4 * 64 * sizeof(v4i) <= sizeof(ChunkLds::v), "query operands exceed the V half of a buffer");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -2048,7 +2049,7 @@ const char *launch_online_int8_rows(Context &c, const View *b, const boot_kernel
     d.rows = (uint32_t)rows;
     d.pos = p.pos;
     d.zs = (uint32_t)((rows + 3) / 4);
-    // One split, or one round of work-groups: a chunk of 128 keys takes about 2.4 us of a work-group,
+    // One split, or one round of work-groups: a chunk of 128 keys takes about 2.5 us of a work-group,
     // the combine 4 us and 0.067 us per row (64 rows after 200 keys: 3 splits 18.0, one 15.2 us; 8
     // rows after 1000: 8 splits 14.0 us, one about 27). More than 64 rows are never split (the
     // combine of 200 rows takes 21 us).
