@@ -563,6 +563,27 @@ __device__ __attribute__((always_inline)) inline void query_parts(const float4 &
 // 1.9e-34) give operands below the full 2^7 instead of an infinite factor.
 constexpr float kLeastVScale = 0x1p-119f;
 
+// The exponents' arguments score - ref of a lane's four tokens. One fma of the dot keeps the product
+// unrounded, but ref is a rounded score: where scores pass 2^20 the rounding it holds (2^-25 of it) would
+// show, and from 2^25 the largest probability no longer fits FP16, or underflows. There the score is
+// rounded first, as the one that ref was taken from; per lane, so that a row does not depend on its
+// neighbours, and behind `large`, which is wave-uniform and changes with the references only.
+__device__ inline bool large_ref(float ref) { return fabsf(ref) > 0x1p20f; }
+
+__device__ __attribute__((always_inline)) inline void exp_args(const float (&dot)[4], float qsc, const float (&ks)[4], float ref,
+                                                               bool large, float (&arg)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) arg[r] = fmaf(dot[r], qsc * ks[r], -ref);
+    if (large) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            float score = dot[r] * (qsc * ks[r]);
+            asm("" : "+v"(score));   // (not contracted into an fma again)
+            arg[r] = large_ref(ref) ? score - ref : arg[r];
+        }
+    }
+}
+
 // One chunk of one KV group in flight, K and V in separate register sets (K is staged
 // one chunk ahead of V): thread t holds K rows t / 16 + 32 i (16 bytes at 16 (t % 16))
 // and V page-row segments t / 8 + 64 i (16 bytes at 16 (t % 8)), i < 4: every load
@@ -887,6 +908,7 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     o[1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     float m = -INFINITY, l = 0.0f, total_prev = 0.0f;   // l: this lane's tokens, summed at the end
     float dot_prev[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // the previous chunk's dots, for a rebuild of its operands
+    bool large = false;   // some column's reference is large (exp_args)
 
     // Probabilities of the lane's four tokens of chunk j against the running reference, as the FP16 hi
     // (column n < 8) or lo (n >= 8) part of p * vs / vs_ref, published as this wave's P operand;
@@ -898,8 +920,7 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
         const float vsr[4] = {vs4.x, vs4.y, vs4.z, vs4.w}, ksr[4] = {ks4.x, ks4.y, ks4.z, ks4.w};
         const float refc = fmaxf(m, -3.0e38f);   // m = -inf only in a column without a score yet
         float arg[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) arg[r] = fmaf(dot_prev[r], qsc * ksr[r], -refc);
+        exp_args(dot_prev, qsc, ksr, refc, large, arg);
         if (begin + (j + 1) * kChunk > end)   // uniform: only a row's last chunk holds tokens past its end
 #pragma unroll
             for (int r = 0; r < 4; r++) arg[r] = begin + local0 + r < end ? arg[r] : -INFINITY;
@@ -939,6 +960,7 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
                 o[0] *= decay;
                 o[1] *= decay;
                 m = next;
+                large = __builtin_amdgcn_ballot_w64(large_ref(m)) != 0;
                 probs(j - 1);   // no wave reads the slot before this branch
                 __syncthreads();
             }
@@ -1401,6 +1423,7 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
 #pragma unroll
         for (int r = 0; r < 4; r++) dot_prev[ct][r] = 0.0f;
     }
+    bool large = false;   // some column's reference is large (exp_args)
     auto probs = [&](uint32_t j) __attribute__((always_inline)) {
         const int slot = j & 1, local0 = (int)(j * kChunk) + 16 * wave + 4 * qq;
         const float4 vs4 = *reinterpret_cast<const float4 *>(&vscale[local0]);
@@ -1413,11 +1436,9 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
             // m = -inf only in a column without a score yet
             const float refc = fmaxf(m[ct], -3.0e38f);
             float arg[4], vf[4], scaled[4];   // vf: the operands' V factors
+            exp_args(dot_prev[ct], qsc[ct], ksr, refc, large, arg);
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                arg[r] = fmaf(dot_prev[ct][r], qsc[ct] * ksr[r], -refc);
-                vf[r] = vsr[r] * vinv[ct];
-            }
+            for (int r = 0; r < 4; r++) vf[r] = vsr[r] * vinv[ct];
             if (edge)   // uniform. A token the row does not see may exceed vref by any factor: its vf too is 0
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
@@ -1467,13 +1488,16 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
         // Chunk 0 has no reference before its maxima: its operands are made here
         if (j == 1 || __builtin_amdgcn_ballot_w64(raise) != 0) {
             float decay[CT];
+            bool any_large = false;
 #pragma unroll
             for (int ct = 0; ct < CT; ct++) {
                 const float next = ctop[ct] > m[ct] + 8.0f ? ctop[ct] : m[ct];
                 decay[ct] = next == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[ct] - next);
                 l[ct] *= decay[ct];
                 m[ct] = next;
+                any_large |= large_ref(next);
             }
+            large = __builtin_amdgcn_ballot_w64(any_large) != 0;
             if constexpr (kWide) {
                 const float first = decay[0], second = decay[CT - 1];
                 ow *= oct ? second : first;
