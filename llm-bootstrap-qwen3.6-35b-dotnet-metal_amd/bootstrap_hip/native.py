@@ -251,7 +251,11 @@ class Device:
             offsets = (ctypes.c_uint64 * max(count, 1))(*(offsets or ()))
         # plain ints of 32 bits pass as they are; anything else (NumPy integers, wider ints) by the
         # declared argument types, which convert or refuse it
-        if type(threads_x) is type(threads_y) is type(group) is int and (threads_x | threads_y | group) >> 32 == 0:
+        try:
+            wide = (threads_x | threads_y | group) >> 32
+        except TypeError:
+            wide = None
+        if type(wide) is int and wide == 0:
             entry = self._entries[1 if noalloc else 0]
         else:
             entry = self.lib.boot_dispatch_noalloc if noalloc else self.lib.boot_dispatch
