@@ -534,11 +534,25 @@ __device__ inline void add_row_partner8(int (&a)[4]) {
     a[3] = r3;
 }
 
+// The largest magnitude of heads whose four dimensions a lane holds, NaN for a head with a NaN (the
+// maximum instructions drop it)
+template <int N>
+__device__ __attribute__((always_inline)) inline void head_max(const float4 (&q)[N], float (&amax)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) amax[i] = fmaxf(fmaxf(fabsf(q[i].x), fabsf(q[i].y)), fmaxf(fabsf(q[i].z), fabsf(q[i].w)));
+    wave_allmax(amax);
+#pragma unroll
+    for (int i = 0; i < N; i++)
+        if (__builtin_amdgcn_ballot_w64(__builtin_isunordered(q[i].x, q[i].y) | __builtin_isunordered(q[i].z, q[i].w)) != 0)
+            amax[i] = __builtin_nanf("");
+}
+
 // The three INT8 parts of four query elements of a head whose largest magnitude is amax, four codes a
 // word. z = q / s_q lies in [-127, 127]; q1 = rint(z), q2 = rint(254 r1) of the remainder r1 = z - q1
 // (|r1| <= 1/2) and q3 = rint(254 r2) of r2 = 254 r1 - q2. Adding 1.5 x 2^23 rounds to an integer
 // whose low byte is its two's complement code: 7 operations an element where rint, clamp, convert and
-// pack took 20 (an instruction of 8 waves on 4 SIMDs: 8 cycles).
+// pack took 20 (an instruction of 8 waves on 4 SIMDs: 8 cycles). A NaN leaves code 0: head_max carries it
+// into the head's scores.
 __device__ __attribute__((always_inline)) inline void query_parts(const float4 &q, float amax, uint32_t (&w)[3]) {
     constexpr float kMagic = 12582912.0f;
     const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
@@ -858,8 +872,9 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     // ---- the INT8 parts of head `wave`, one lane's four dimensions (as rows_int8_kernel: each wave
     // one head, where every wave built a quarter of all eight and the maxima met behind a barrier)
     {
-        float amax[1] = {fmaxf(fmaxf(fabsf(rq.x), fabsf(rq.y)), fmaxf(fabsf(rq.z), fabsf(rq.w)))};
-        wave_allmax(amax);
+        const float4 x[1] = {rq};
+        float amax[1];
+        head_max(x, amax);
         uint32_t w[3];
         query_parts(rq, amax[0], w);
         const int c = lane >> 4, bq = (lane >> 2) & 3, mix = 4 * c + bq;
@@ -1340,9 +1355,7 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
 
     // ---- the query's INT8 parts
     float amax[kRowsPer];
-#pragma unroll
-    for (int r = 0; r < kRowsPer; r++) amax[r] = fmaxf(fmaxf(fabsf(x[r].x), fabsf(x[r].y)), fmaxf(fabsf(x[r].z), fabsf(x[r].w)));
-    wave_allmax(amax);
+    head_max(x, amax);
 #pragma unroll
     for (int r = 0; r < kRowsPer; r++) {
         uint32_t w[3];

@@ -1,6 +1,6 @@
 """Scores far beyond any softmax in use (K scales times 2^14 to 2^100): the probability operands stay
 finite and a row returns the value of its largest score, on the kernels that take the exponents'
-arguments from the dots."""
+arguments from the dots; a NaN in a query reaches its head's output and no other."""
 import numpy as np
 import pytest
 
@@ -39,3 +39,16 @@ def test_large_scores(device, oracle, kind, history, rows, power):
     assert np.all(np.isfinite(y))
     ref = oracle.attention(q, *host, gate, rows, history, round_q_half=int(kind == "prefill"))
     assert rel_l2(y, ref) <= (REL_L2 if kind == "prefill" else 5e-6)
+
+
+@pytest.mark.parametrize("kind,history,rows", CASES)
+def test_nan_query(device, oracle, kind, history, rows):
+    """The head holding the NaN is NaN as the reference's float arithmetic has it; every other head is
+    bitwise what it is without."""
+    q, gate, host = build_case(oracle, history, rows)
+    plain = run(device, kind, q, gate, host, rows, history).reshape(rows, 16, 256)
+    q.reshape(rows, 16, 256)[rows // 2, 3, 7] = np.nan
+    y = run(device, kind, q, gate, host, rows, history).reshape(rows, 16, 256)
+    assert np.all(np.isnan(y[rows // 2, 3]))
+    y[rows // 2, 3] = plain[rows // 2, 3]
+    assert np.array_equal(y.view(np.uint32), plain.view(np.uint32))
