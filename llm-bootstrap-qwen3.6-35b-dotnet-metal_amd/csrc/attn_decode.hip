@@ -577,6 +577,17 @@ __device__ __attribute__((always_inline)) inline void query_parts(const float4 &
 // 1.9e-34) give operands below the full 2^7 instead of an infinite factor.
 constexpr float kLeastVScale = 0x1p-119f;
 
+// A split's result is (m, l, O) for l 2^m and O 2^m: O, the sum of up to 2^40 (p <= 2^8, codes and the
+// operands' 2^7, 2^18 keys) times the V scale, would pass FP32 where the scale is large, so its factor,
+// l's and 2^-m's are then 2^-40 each. (The outputs divide O by l.)
+constexpr float kLargeVScale = 0x1p60f;
+__device__ inline void shift_large_values(float &vs_out, float &l, float &m) {
+    const bool shift = vs_out > kLargeVScale;
+    vs_out *= shift ? 0x1p-40f : 1.0f;
+    l *= shift ? 0x1p-40f : 1.0f;
+    m += shift ? 40.0f : 0.0f;
+}
+
 // The exponents' arguments score - ref of a lane's four tokens. One fma of the dot keeps the product
 // unrounded, but ref is a rounded score: where scores pass 2^20 the rounding it holds (2^-25 of it) would
 // show, and from 2^25 the largest probability no longer fits FP16, or underflows. There the score is
@@ -1086,6 +1097,7 @@ __global__ __launch_bounds__(512, 1) void decode_int8_kernel(DecodeParams p) {
     // results as inline-assembly operands, for which the compiler inserts no wait states:
     // cover them here), then lanes n < 8 hold tile 2 wave and lanes n >= 8 tile 2 wave + 1.
     l = xl_sum32(xl_sum16(l));
+    shift_large_values(vs_ref, l, m);
     if (qq == 0) wave_l[wave][n] = l;
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
@@ -1663,7 +1675,8 @@ __global__ __launch_bounds__(512, 1) void rows_int8_kernel(RowsParams p) {
     // ---- O^T[d][n] times the column's V scale reference, l over the lanes and waves
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) {
-        const float lt = xl_sum32(xl_sum16(l[ct]));
+        float lt = xl_sum32(xl_sum16(l[ct]));
+        shift_large_values(vref[ct], lt, m[ct]);
         if (qq == 0) wave_l[ct][wave][n] = lt;
     }
     // the lane's quads of O, four dimensions of one column each: tile, first dimension, values

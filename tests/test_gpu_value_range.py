@@ -1,6 +1,7 @@
-"""V vectors near the bottom of FP32's range on the kernels that scale the probability operands by a
+"""V vectors near either end of FP32's range on the kernels that scale the probability operands by a
 split's largest V scale: a split (or a row's whole range) of vectors around 1e-36 beside ordinary
-ones, alone, and before a later token whose V a row does not see."""
+ones, alone, and before a later token whose V a row does not see; and vectors around 3e38, whose sums
+before the division by the softmax's denominator lie beyond FP32, alone, in one split and in one token."""
 import numpy as np
 import pytest
 
@@ -44,5 +45,28 @@ def test_tiny_values(device, oracle, kind, history, rows, where):
     ref = oracle.attention(q, *host, gate, rows, history, round_q_half=int(kind == "prefill"))
     for r, (a, b) in enumerate(zip(y.reshape(rows, 4096), np.asarray(ref).reshape(rows, 4096))):
         scale = np.abs(b).max()   # (norms of values around 1e-37 would underflow)
+        assert rel_l2(a.astype(np.float64) / scale, b / scale) <= (REL_L2 if kind == "prefill" else 5e-6), r
+    cache.dispose()
+
+
+@pytest.mark.parametrize("where", ["split", "all", "last"])
+@pytest.mark.parametrize("kind,history,rows", [
+    ("decode", 200, 1), ("decode", 4092, 1), ("decode", 1000, 5), ("prefill", 1000, 16), ("prefill", 0, 98),
+    ("prefill", 2031, 18), ("verify", 300, 2), ("verify", 1500, 8)])
+def test_huge_values(device, oracle, kind, history, rows, where):
+    """Flat rows (queries a tenth of the others') against FP64, each row at the bounds above."""
+    keys, values = reference_kv(history + rows)
+    values[{"split": slice(128, 256), "all": slice(None), "last": slice(-1, None)}[where]] *= np.float32(3e38)
+    q, gate, host = build_case(oracle, history, rows, kv=(keys, values))
+    q = q * np.float32(0.1)
+    cache = upload_cache(device, *host)
+    if kind == "verify":
+        y = verify(device, q, gate, cache, rows, history)
+    else:
+        y = (run_decode if kind == "decode" else run_prefill)(device, q, gate, cache, rows, history)[:-1]
+    assert np.all(np.isfinite(y))
+    ref = oracle.attention(q, *host, gate, rows, history, round_q_half=int(kind == "prefill"))
+    for r, (a, b) in enumerate(zip(y.reshape(rows, 4096), np.asarray(ref).reshape(rows, 4096))):
+        scale = np.abs(b).max()
         assert rel_l2(a.astype(np.float64) / scale, b / scale) <= (REL_L2 if kind == "prefill" else 5e-6), r
     cache.dispose()
